@@ -587,7 +587,7 @@ def run_prefill(torch, q4k, args):
     jobs = [(wh, A[t].float().cpu().numpy(), np.empty(n, np.float32), n, bpr) for t in range(toks)]
     return {"workload": f"config5: prefill 18944x3584 Q4_K x f16 [512x3584], {copies} weight copies",
             "us_per_launch": round(s * 1e6, 3), "tflops": tflops, "parity": parity,
-            "kernel": "mgq::gemm_q4k_f16_lds_kernel",
+            "kernel": "mgq::gemm_q4k_f16_kernel",
             "cpu": (jobs, 2.0 * n * k * toks / 1e12, "TFLOP/s",
                     f"{toks} of the 512 tokens, one CPU matvec each (2*N*K flops per token)", 5)}
 

@@ -1,0 +1,120 @@
+"""The prefill GEMM's tile shapes: one case or more for each, at their edges
+(one row, one token, a tile's rows and tokens +- 1, K shares with and without
+a block), pointers of the smallest alignment, and recording into a graph.
+
+Bounds as for the other GEMM tests: f16 weights (three roundings of 2^-11
+each) keep the Frobenius error below 1e-3 and each element within
+1e-2 sum|w||a| / sqrt(K)."""
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from modgrad_amd import _lib
+from tests.gpu_util import dev, empty_f32, host, ptr, random_q4k_bytes
+
+pytestmark = pytest.mark.gpu
+
+def note(msg: str) -> None:
+    print(f"[case] {msg}", flush=True)
+
+
+@pytest.fixture(scope="module")
+def L():
+    return _lib.load()
+
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def check(L, orc, n, bpr, m, woff=0, aoff=0, coff=0):
+    rng = np.random.default_rng(n + 17 * bpr + 1009 * m + woff)
+    w = random_q4k_bytes(rng, n * bpr)
+    a = rng.standard_normal((m, bpr * 256)).astype(np.float16)
+    wt = dev(np.concatenate([np.zeros(woff, np.uint8), w]))
+    at = dev(np.concatenate([np.zeros(aoff, np.uint8), a.view(np.uint8).ravel()]))
+    ct = empty_f32(m * n + coff // 4)
+    _lib.check("gemm", L.launch_gemm_q4k_f16(ptr(wt) + woff, ptr(at) + aoff, ptr(ct) + coff, n, bpr,
+                                             m, None))
+    rows = None
+    if n > 600:
+        rows = np.unique(np.concatenate([rng.choice(n, size=160, replace=False),
+                                         np.arange(48), np.arange(n - 48, n)])).astype(np.int32)
+    C = host(ct)[coff // 4:].reshape(m, n)
+    assert np.all(np.isfinite(C))
+    C = C if rows is None else C[:, rows]
+    C_ref, A = orc.gemm_f16(w, a.view(np.uint16), n, bpr, rows=rows)
+    assert np.all(np.abs(C - C_ref) <= 1e-2 * A / np.sqrt(bpr * 256))
+    assert np.linalg.norm(C - C_ref) <= 1e-3 * np.linalg.norm(C_ref)
+
+
+@pytest.mark.parametrize("n,bpr,m", [
+    (1, 1, 1), (17, 3, 16), (33, 5, 15), (1000, 6, 17),           # 32 x 16, four K shares
+    (1000, 1, 129), (4001, 9, 33),                                # 32 x 32
+    (2001, 1, 129), (8003, 5, 33),                                # 32 x 48
+    (16001, 1, 1), (16001, 3, 49), (4001, 3, 129),                # 64 x 48, two K shares
+    (8003, 2, 97), (16001, 3, 81),                                # 64 x 80
+    (20479, 2, 1), (30001, 2, 47),                                # 128 x 48
+    (30001, 1, 49), (16001, 3, 97),                               # 128 x 64
+    (16001, 2, 129), (30001, 1, 79),                              # 128 x 80
+    (20479, 1, 17), (30001, 3, 47),                               # 160 x 48
+    (37888, 26, 33),                                              # 160 x 48, two K shares
+    (20479, 2, 127), (20479, 3, 97),                              # 160 x 80
+    (42001, 1, 5), (42001, 3, 127),                               # 224 x 128
+    (60001, 2, 1), (85007, 3, 79),                                # 336 x 80
+    (30001, 1, 161), (85007, 2, 81), (60001, 3, 127)])            # 336 x 128
+def test_gemm_tile_shapes(L, orc, n, bpr, m):
+    note(f"gemm tiles n={n} bpr={bpr} m={m}")
+    check(L, orc, n, bpr, m)
+
+
+# weights at an odd byte, activations at an odd f16, C at a 4-byte address:
+# the token copies then go through registers
+@pytest.mark.parametrize("n,bpr,m", [(100, 3, 33), (2001, 5, 129), (30001, 3, 161)])
+@pytest.mark.parametrize("woff,aoff,coff", [(1, 0, 0), (0, 2, 4), (3, 10, 8)])
+def test_gemm_unaligned_pointers(L, orc, n, bpr, m, woff, aoff, coff):
+    note(f"gemm n={n} bpr={bpr} m={m} offsets {woff} {aoff} {coff}")
+    check(L, orc, n, bpr, m, woff, aoff, coff)
+
+
+CAPTURE = """
+import ctypes, sys, torch
+sys.path.insert(0, sys.argv[1])
+from modgrad_amd import _lib
+L = _lib.load()
+gen = torch.Generator(device="cuda"); gen.manual_seed(5)
+jobs = []
+for n, bpr, m in ((1000, 6, 17), (8003, 2, 97), (30001, 1, 161)):
+    w = torch.randint(0, 256, (n * bpr, 144), dtype=torch.uint8, device="cuda", generator=gen)
+    w[:, :4] = torch.full((n * bpr, 2), 1e-3, device="cuda").half().view(torch.uint8)
+    a = torch.randn(m, bpr * 256, device="cuda", generator=gen).half()
+    jobs.append((w, a, torch.zeros(m, n, device="cuda"), n, bpr, m))
+torch.cuda.synchronize()
+def run(stream):
+    for w, a, c, n, bpr, m in jobs:
+        assert L.launch_gemm_q4k_f16(w.data_ptr(), a.data_ptr(), c.data_ptr(), n, bpr, m,
+                                     ctypes.c_void_p(stream)) == 0
+g = torch.cuda.CUDAGraph()
+with torch.cuda.graph(g):  # the library's first call in this process
+    run(torch.cuda.current_stream().cuda_stream)
+for i in range(4):
+    for j in jobs:
+        j[1].copy_(torch.randn(j[1].shape, device="cuda", generator=gen).half())
+        j[2].fill_(float("nan"))
+    g.replay()
+    torch.cuda.synchronize()
+    got = [j[2].clone() for j in jobs]
+    run(0)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, j[2]) for a, j in zip(got, jobs)), i
+print("replays equal")
+"""
+
+
+def test_gemm_first_call_in_a_graph():
+    note("gemm recorded into a graph as the library's first call, 4 replays")
+    r = subprocess.run([sys.executable, "-c", CAPTURE, ROOT], capture_output=True, text=True,
+                       timeout=110)
+    assert r.returncode == 0 and "replays equal" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
