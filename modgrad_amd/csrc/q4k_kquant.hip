@@ -261,6 +261,8 @@ hipError_t gemv_q6k_launch(const uint8_t *w, const float *x, float *y, int n, in
 
 hipError_t gemv_q6k_q8_launch(const uint8_t *w, const int8_t *xq, const float *xd, float *y,
                               int n, int bpr, hipStream_t stream) {
+    const hipError_t e = gemv_q6k_q8_mfma_launch(w, xq, xd, y, n, bpr, stream);
+    if (e != hipErrorNotSupported) return e;
     gemv_q6k_q8_kernel<<<(unsigned)((n + 3) / 4), 256, 0, stream>>>(w, xq, xd, y, n, bpr);
     return hipGetLastError();
 }

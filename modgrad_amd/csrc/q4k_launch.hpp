@@ -227,6 +227,11 @@ hipError_t gemv_q6k_mfma_launch(const uint8_t *w, const float *x, float *y, int 
 hipError_t gemv_q6k_mfma_norm_launch(const uint8_t *w, const float *x, const float *nw, float eps,
                                      float *y, int n, int bpr, hipStream_t stream);
 
+// Q6_K on Q8_1 activations on the matrix cores; hipErrorNotSupported as for
+// gemv_q6k_mfma_launch, or when the row's table does not fit LDS.
+hipError_t gemv_q6k_q8_mfma_launch(const uint8_t *w, const int8_t *xq, const float *xd, float *y,
+                                   int n, int bpr, hipStream_t stream);
+
 // Q5_K / Q6_K matvecs (f32 activations) and Q6_K on Q8_1 activations.
 hipError_t gemv_q5k_launch(const uint8_t *w, const float *x, float *y, int n, int bpr,
                            hipStream_t stream);

@@ -128,6 +128,34 @@ __device__ __forceinline__ void q6m_item(uint8_t *lds, float *meta, int i, bool 
     *reinterpret_cast<u32x4 *>(ent + 16) = hl;
 }
 
+// q6m_item on Q8_1 activations: the int8 values of item i are exact in f16, so
+// the table holds them as they are (no xl part) and the products of a half
+// (at most 63 * 127 * 16) stay exact integers in the f32 accumulators. meta
+// holds the sub-block's scale xd and the integer sums of its halves.
+__device__ __forceinline__ void q6m_item_q8(uint8_t *lds, float *meta, int i, bool valid, u32x2 xq, float xd) {
+    using namespace q6m;
+    float v[8], sum = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const uint32_t d = q < 4 ? xq[0] : xq[1];
+        v[q] = (float)(int8_t)(d >> (8 * (q & 3)));
+        sum += v[q];
+    }
+    sum += quad_xor<1>(sum);  // the 16 values of this half
+    if (!valid) return;
+    const int b = i >> 5, j = (i >> 2) & 7, kg = i & 3;
+    if (kg == 0) meta[b * META + j] = xd;
+    if ((kg & 1) == 0) meta[b * META + 8 + 2 * j + (kg >> 1)] = sum;
+    const float xs[8] = {v[0], v[2], v[1], v[3], v[4], v[6], v[5], v[7]};
+    u32x4 hh;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        hh[q] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(xs[2 * q], xs[2 * q + 1]));
+    uint8_t *ent = lds + (size_t)b * TAB + (size_t)((j * 4 + kg) * 2) * 16;
+    *reinterpret_cast<u32x4 *>(ent) = hh;
+    *reinterpret_cast<u32x4 *>(ent + 16) = u32x4{0u, 0u, 0u, 0u};
+}
+
 // Lane (n16, g) supplies A row n16, k-slice g of every MFMA. Row n16 is
 // nonzero only in the MFMAs of sub-blocks c with c % 4 = n16 / 4, and only in
 // its half's k-slices (g / 2 = (n16 / 2) % 2): there it is table entry
@@ -150,6 +178,9 @@ __device__ __forceinline__ Q6mLane q6m_lane(int lane) {
 // 32 (sc X_0 + sc X_1)) over its sub-blocks g and 4 + g. aop holds the A
 // operands: zero (set once by the caller) except where the lane's row is
 // nonzero, which only those lanes reload, block by block.
+// Q8 (table from q6m_item_q8): d * sum_j xd_j (sc i_0 + sc i_1), i_h the exact
+// integer dot of half h.
+template <bool Q8 = false>
 __device__ __forceinline__ float q6m_block(const uint8_t *lds, const uint8_t *stage, uint32_t rb,
                                            int b, Q6mLane ln, half8 (&aop)[8], const float *meta,
                                            int g) {
@@ -210,6 +241,12 @@ __device__ __forceinline__ float q6m_block(const uint8_t *lds, const uint8_t *st
         const float sc0 = (float)(int8_t)stage[rb + 192 + 2 * j];
         const float sc1 = (float)(int8_t)stage[rb + 193 + 2 * j];
         const float s0 = acc[a][0] + acc[a][1], s1 = acc[a][2] + acc[a][3];
+        if constexpr (Q8) {
+            const float up = (j & 2) ? 1048576.0f : 16777216.0f;  // the operands' 2^-20 or 2^-24
+            const float i0 = s0 * up - 32.0f * mb[8 + 2 * j], i1 = s1 * up - 32.0f * mb[9 + 2 * j];
+            y += mb[j] * d * (sc0 * i0 + sc1 * i1);
+            continue;
+        }
         y += d * (mb[j] * (sc0 * s0 + sc1 * s1) - 32.0f * (sc0 * mb[8 + 2 * j] + sc1 * mb[9 + 2 * j]));
     }
     return y;
@@ -464,14 +501,19 @@ __host__ __device__ inline Q6mLayout q6w_layout(int bpr, int rounds, int nw) {
     return L;
 }
 
-template <int NW, int XI, bool NORM = false>
+// XM: kX32 (f32 x), kXNorm (its fused RMSNorm) or kXQ8 (Q8_1 activations xq, xd)
+constexpr int kX32 = 0, kXNorm = 1, kXQ8 = 2;
+template <int NW, int XI, int XM = kX32>
 __global__ __launch_bounds__(NW * 64) void gemv_q6k_wave_long_kernel(const uint8_t *__restrict__ w,
                                                                      const float *__restrict__ x,
                                                                      float *__restrict__ y, int n,
                                                                      int bpr, int rounds,
                                                                      GemvSched sch,
                                                                      const float *__restrict__ nw = nullptr,
-                                                                     float eps = 0.0f) {
+                                                                     float eps = 0.0f,
+                                                                     const int8_t *__restrict__ xq = nullptr,
+                                                                     const float *__restrict__ xd = nullptr) {
+    constexpr bool NORM = XM == kXNorm, Q8 = XM == kXQ8;
     using q6m::R, q6m::BB, q6m::TAB;
     using q6w::CH, q6w::PITCH, q6w::UP, q6w::IPU;
     constexpr int NT = NW * 64;
@@ -526,35 +568,49 @@ __global__ __launch_bounds__(NW * 64) void gemv_q6k_wave_long_kernel(const uint8
 
     // ---- prologue: the whole row's activation table, XI items per thread ---
     const int nitems = bpr * 32;
-    f32x4 xv[2 * XI];
-#pragma unroll
-    for (int k = 0; k < XI; ++k) {
-        const int ii = min(tid + k * NT, nitems - 1);
-        xv[2 * k] = ld_f32x4(x + (size_t)ii * 8);
-        xv[2 * k + 1] = ld_f32x4(x + (size_t)ii * 8 + 4);
-    }
     float *normp = reinterpret_cast<float *>(lds + Lo.normp);
-    if constexpr (NORM) {
-        // sum(x^2) of this thread's items (clamped duplicates add 0), reduced
-        // per wavefront; the table holds x .* nw (as gemv_q6k_mfma_kernel)
-        float ssq = 0.0f;
+    if constexpr (Q8) {
+        u32x2 qv[XI];
+        float dv[XI];
 #pragma unroll
         for (int k = 0; k < XI; ++k) {
-            const f32x4 v0 = xv[2 * k], v1 = xv[2 * k + 1];
-            const float s = ((v0[0] * v0[0] + v0[1] * v0[1]) + (v0[2] * v0[2] + v0[3] * v0[3])) +
-                            ((v1[0] * v1[0] + v1[1] * v1[1]) + (v1[2] * v1[2] + v1[3] * v1[3]));
-            ssq += tid + k * NT < nitems ? s : 0.0f;
             const int ii = min(tid + k * NT, nitems - 1);
-            xv[2 * k] = v0 * ld_f32x4(nw + (size_t)ii * 8);
-            xv[2 * k + 1] = v1 * ld_f32x4(nw + (size_t)ii * 8 + 4);
+            qv[k] = *reinterpret_cast<const u32x2_a1 *>(xq + (size_t)ii * 8);
+            dv[k] = xd[ii >> 2];
         }
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) ssq += __shfl_xor(ssq, off, 64);
-        if (lane == 0) normp[wave] = ssq;
-    }
+        for (int k = 0; k < XI; ++k)
+            q6m_item_q8(lds, meta, tid + k * NT, tid + k * NT < nitems, qv[k], dv[k]);
+    } else {
+        f32x4 xv[2 * XI];
 #pragma unroll
-    for (int k = 0; k < XI; ++k)
-        q6m_item(lds, meta, tid + k * NT, tid + k * NT < nitems, xv[2 * k], xv[2 * k + 1]);
+        for (int k = 0; k < XI; ++k) {
+            const int ii = min(tid + k * NT, nitems - 1);
+            xv[2 * k] = ld_f32x4(x + (size_t)ii * 8);
+            xv[2 * k + 1] = ld_f32x4(x + (size_t)ii * 8 + 4);
+        }
+        if constexpr (NORM) {
+            // sum(x^2) of this thread's items (clamped duplicates add 0), reduced
+            // per wavefront; the table holds x .* nw (as gemv_q6k_mfma_kernel)
+            float ssq = 0.0f;
+#pragma unroll
+            for (int k = 0; k < XI; ++k) {
+                const f32x4 v0 = xv[2 * k], v1 = xv[2 * k + 1];
+                const float s = ((v0[0] * v0[0] + v0[1] * v0[1]) + (v0[2] * v0[2] + v0[3] * v0[3])) +
+                                ((v1[0] * v1[0] + v1[1] * v1[1]) + (v1[2] * v1[2] + v1[3] * v1[3]));
+                ssq += tid + k * NT < nitems ? s : 0.0f;
+                const int ii = min(tid + k * NT, nitems - 1);
+                xv[2 * k] = v0 * ld_f32x4(nw + (size_t)ii * 8);
+                xv[2 * k + 1] = v1 * ld_f32x4(nw + (size_t)ii * 8 + 4);
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) ssq += __shfl_xor(ssq, off, 64);
+            if (lane == 0) normp[wave] = ssq;
+        }
+#pragma unroll
+        for (int k = 0; k < XI; ++k)
+            q6m_item(lds, meta, tid + k * NT, tid + k * NT < nitems, xv[2 * k], xv[2 * k + 1]);
+    }
     // a wavefront with no blocks contributes zero rows
     if (nb == 0)
         for (int i = lane; i < my_groups * R; i += 64) aux[((i / R) * NW + wave) * R + i % R] = 0.0f;
@@ -587,7 +643,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_q6k_wave_long_kernel(const uint8
         const int b = wave + k * NW;
         const int row = min(sched_group(sch, (int)blockIdx.x, (int)gridDim.x, q) * R + n16, n - 1);
         const uint32_t rb = (uint32_t)(n16 * PITCH * 16) + (uint32_t)(((long)row * RB + (long)b * BB) & 15);
-        yacc += q6m_block(lds, slot, rb, b, ln, aop, meta, g);
+        yacc += q6m_block<Q8>(lds, slot, rb, b, ln, aop, meta, g);
         if (++k == nb) {
             yacc += __shfl_xor(yacc, 16, 64);
             yacc += __shfl_xor(yacc, 32, 64);
@@ -658,26 +714,27 @@ hipError_t q6m_long_launch(const uint8_t *w, const float *x, float *y, int n, in
                       q6m_long_probe<NW, XI>(), stream);
 }
 
-template <int NW, int XI, bool NORM = false>
+template <int NW, int XI, int XM = kX32>
 hipError_t q6w_long_setup(int *occ) {
-    const void *kern = (const void *)gemv_q6k_wave_long_kernel<NW, XI, NORM>;
+    const void *kern = (const void *)gemv_q6k_wave_long_kernel<NW, XI, XM>;
     const hipError_t attr = allow_full_lds_by_addr(kern);
     if (attr != hipSuccess) return attr;
     *occ = occupancy_cached(kern, NW * 64, q6w_layout(q6m_long_probe<NW, XI>(), 8, NW).total, 1);
     return hipSuccess;
 }
 
-template <int NW, int XI, bool NORM = false>
+template <int NW, int XI, int XM = kX32>
 hipError_t q6w_long_launch(const uint8_t *w, const float *x, float *y, int n, int bpr,
-                           hipStream_t stream, const float *nw = nullptr, float eps = 0.0f) {
+                           hipStream_t stream, const float *nw = nullptr, float eps = 0.0f,
+                           const int8_t *xq = nullptr, const float *xd = nullptr) {
     int occ = 1;
-    const hipError_t attr = q6w_long_setup<NW, XI, NORM>(&occ);
+    const hipError_t attr = q6w_long_setup<NW, XI, XM>(&occ);
     if (attr != hipSuccess) return attr;
     const PersistPlan p = persistent_plan((n + q6m::R - 1) / q6m::R, occ);
     const size_t lds = q6w_layout(bpr, (int)p.rounds, NW).total;
     if (lds > 160 * 1024) return hipErrorNotSupported;
-    gemv_q6k_wave_long_kernel<NW, XI, NORM><<<(unsigned)p.grid, NW * 64, lds, stream>>>(
-        w, x, y, n, bpr, (int)p.rounds, p.sch, nw, eps);
+    gemv_q6k_wave_long_kernel<NW, XI, XM><<<(unsigned)p.grid, NW * 64, lds, stream>>>(
+        w, x, y, n, bpr, (int)p.rounds, p.sch, nw, eps, xq, xd);
     return hipGetLastError();
 }
 
@@ -707,7 +764,10 @@ hipError_t q6k_prepare() {
     if (e == hipSuccess) e = q6w_long_setup<LONG_NW, 4>(&occ);
     if (e == hipSuccess) e = q6w_long_setup<LONG_NW, 6>(&occ);
     if (e == hipSuccess) e = q6w_long_setup<LONG_NW, 8>(&occ);
-    if (e == hipSuccess) e = q6w_long_setup<14, 1, true>(&occ);
+    if (e == hipSuccess) e = q6w_long_setup<14, 1, kXNorm>(&occ);
+    if (e == hipSuccess) e = q6w_long_setup<14, 1, kXQ8>(&occ);
+    if (e == hipSuccess) e = q6w_long_setup<LONG_NW, 2, kXQ8>(&occ);
+    if (e == hipSuccess) e = q6w_long_setup<LONG_NW, 4, kXQ8>(&occ);
     return e;
 }
 
@@ -752,6 +812,22 @@ hipError_t gemv_q6k_mfma_launch(const uint8_t *w, const float *x, float *y, int 
     return hipErrorNotSupported;
 }
 
+// Q6_K on Q8_1 activations (launch_matvec_q6k_dp4a) on the wave-private
+// kernel. 3584 x 18944: 194 -> 15.9 us, against the byte-loading vector-ALU
+// kernel that serves what this one cannot take (bpr > 91, misaligned or
+// unpadded weights).
+hipError_t gemv_q6k_q8_mfma_launch(const uint8_t *w, const int8_t *xq, const float *xd, float *y,
+                                   int n, int bpr, hipStream_t stream) {
+    using namespace q6m;
+    if (((uintptr_t)w & 15u) || (((long)n * bpr * BB) % 16)) return hipErrorNotSupported;
+    if (bpr <= MAX_BPR)
+        return q6w_long_launch<14, 1, kXQ8>(w, nullptr, y, n, bpr, stream, nullptr, 0.0f, xq, xd);
+    const int need = (bpr * 32 + LONG_NW * 64 - 1) / (LONG_NW * 64);  // table items per thread
+    if (need <= 2) return q6w_long_launch<LONG_NW, 2, kXQ8>(w, nullptr, y, n, bpr, stream, nullptr, 0.0f, xq, xd);
+    if (need <= 4) return q6w_long_launch<LONG_NW, 4, kXQ8>(w, nullptr, y, n, bpr, stream, nullptr, 0.0f, xq, xd);
+    return hipErrorNotSupported;
+}
+
 hipError_t gemv_q6k_mfma_norm_launch(const uint8_t *w, const float *x, const float *nw, float eps,
                                      float *y, int n, int bpr, hipStream_t stream) {
     using namespace q6m;
@@ -770,7 +846,7 @@ hipError_t gemv_q6k_mfma_norm_launch(const uint8_t *w, const float *x, const flo
         return (v && *v) ? std::atoi(v) : 1;
     }();
     if (whole_env) {
-        const hipError_t ew = q6w_long_launch<14, 1, true>(w, x, y, n, bpr, stream, nw, eps);
+        const hipError_t ew = q6w_long_launch<14, 1, kXNorm>(w, x, y, n, bpr, stream, nw, eps);
         if (ew != hipErrorNotSupported) return ew;
     }
     return q6m_launch(gemv_q6k_mfma_kernel<true>, false, NW, w, x, y, n, bpr, MAX_BPR, stream, nw,
