@@ -116,6 +116,17 @@ hipError_t launch_matvec_q4k_ex(const unsigned char *w_q4, const float *x, float
                                 int out_dim, int k_elems, int layout,
                                 hipStream_t stream);
 
+/* y = W x + bias: launch_matvec_q4k_ex followed by launch_residual_add_ex of
+ * the out_dim floats of bias (the resident linear layer's hipblasSgemv with
+ * beta = 1 on a bias-filled y, rocm.rs:2000-2056), same bits. One launch for
+ * the flattened layout with whole sub-blocks per row (k_elems % 32 == 0,
+ * k_elems % 256 != 0), else the two. y must not overlap bias, x or w.
+ * hipErrorInvalidValue as for launch_matvec_q4k_ex, or for a null or
+ * misaligned bias. */
+hipError_t launch_matvec_q4k_bias_ex(const unsigned char *w_q4, const float *x, const float *bias,
+                                     float *y, int out_dim, int k_elems, int layout,
+                                     hipStream_t stream);
+
 /* launch_quantize_q8_1 / launch_matvec_q4k_dp4a with an explicit stream. */
 hipError_t launch_quantize_q8_1_ex(const float *x, signed char *xq, float *xd, float *xsum, int n,
                                    hipStream_t stream);

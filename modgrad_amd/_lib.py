@@ -26,6 +26,7 @@ SIGNATURES = {
     "launch_dequant_q4k": (I, [P, I, P]),
     "launch_matvec_q4k": (I, [P, P, P, I, I]),
     "launch_matvec_q4k_ex": (I, [P, P, P, I, I, I, P]),
+    "launch_matvec_q4k_bias_ex": (I, [P, P, P, P, I, I, I, P]),
     "launch_quantize_q8_1": (I, [P, P, P, P, I]),
     "launch_matvec_q5k": (I, [P, P, P, I, I]),
     "launch_matvec_q6k": (I, [P, P, P, I, I]),

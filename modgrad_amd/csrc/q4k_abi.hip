@@ -55,6 +55,19 @@ hipError_t launch_matvec_q4k_ex(const unsigned char *w_q4, const float *x, float
     return hipErrorInvalidValue;
 }
 
+hipError_t launch_matvec_q4k_bias_ex(const unsigned char *w_q4, const float *x, const float *bias,
+                                     float *y, int out_dim, int k_elems, int layout,
+                                     hipStream_t stream) {
+    if (!bias || misaligned4(bias)) return hipErrorInvalidValue;
+    if (layout == MGQ_LAYOUT_FLAT && out_dim > 0 && k_elems > 0 && k_elems % 256 != 0 &&
+        ((int64_t)out_dim * k_elems) % 256 == 0 && w_q4 && x && y && !misaligned4(x) && !misaligned4(y)) {
+        const hipError_t e = mgq::gemv_flat_launch(w_q4, x, y, out_dim, k_elems, stream, bias);
+        if (e != hipErrorNotSupported) return e;
+    }
+    const hipError_t e = launch_matvec_q4k_ex(w_q4, x, y, out_dim, k_elems, layout, stream);
+    return e != hipSuccess ? e : launch_residual_add_ex(y, bias, out_dim, stream);
+}
+
 hipError_t launch_matvec_q4k(const unsigned char *w_q4, const float *x, float *y, int out_dim,
                              int blocks_per_row) {
     if (out_dim <= 0 || blocks_per_row <= 0) return hipErrorInvalidValue;

@@ -106,11 +106,15 @@ __global__ __launch_bounds__(256) void gemv_generic_kernel(const uint8_t *__rest
 // nibbles of sub-block 2(j/2) and the 16 high nibbles of sub-block 2(j/2)+1,
 // with 16-byte loads of the 16 matching x values each. Per sub-block half:
 // d*sc * sum(q x) - dmin*m * sum(x), added to the accumulator of its row.
+// bias (may be null): added to the finished row sum, one rounding, as a
+// residual_add launch behind it would (4864x896: that launch and its gap took
+// 2-4 us of a linear layer's 8.7).
 template <int U>
 __global__ __launch_bounds__(256) void gemv_flat_kernel(const uint8_t *__restrict__ w,
                                                         const float *__restrict__ x,
                                                         float *__restrict__ y, int n, int k,
-                                                        int bpu, int units, int64_t nblocks) {
+                                                        int bpu, int units, int64_t nblocks,
+                                                        const float *__restrict__ bias) {
     const int lane = threadIdx.x & 63;
     const int u = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (u >= units) return;  // uniform per wavefront
@@ -156,12 +160,12 @@ __global__ __launch_bounds__(256) void gemv_flat_kernel(const uint8_t *__restric
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
         const int row = u * U + r;
-        if (lane == 0 && row < n) y[row] = v;
+        if (lane == 0 && row < n) y[row] = bias ? v + bias[row] : v;
     }
 }
 
 hipError_t gemv_flat_launch(const uint8_t *w, const float *x, float *y, int n, int k,
-                            hipStream_t stream) {
+                            hipStream_t stream, const float *bias) {
     if (k % 32 != 0) return hipErrorNotSupported;
     int g = 256;
     while (k % g) g >>= 1;  // gcd(k, 256), >= 32 here
@@ -172,10 +176,10 @@ hipError_t gemv_flat_launch(const uint8_t *w, const float *x, float *y, int n, i
     const int64_t nblocks = (int64_t)n * k / kBlockElems;
     const unsigned grid = (unsigned)((units + 3) / 4);
     switch (U) {
-    case 1: gemv_flat_kernel<1><<<grid, 256, 0, stream>>>(w, x, y, n, k, bpu, units, nblocks); break;
-    case 2: gemv_flat_kernel<2><<<grid, 256, 0, stream>>>(w, x, y, n, k, bpu, units, nblocks); break;
-    case 4: gemv_flat_kernel<4><<<grid, 256, 0, stream>>>(w, x, y, n, k, bpu, units, nblocks); break;
-    default: gemv_flat_kernel<8><<<grid, 256, 0, stream>>>(w, x, y, n, k, bpu, units, nblocks); break;
+    case 1: gemv_flat_kernel<1><<<grid, 256, 0, stream>>>(w, x, y, n, k, bpu, units, nblocks, bias); break;
+    case 2: gemv_flat_kernel<2><<<grid, 256, 0, stream>>>(w, x, y, n, k, bpu, units, nblocks, bias); break;
+    case 4: gemv_flat_kernel<4><<<grid, 256, 0, stream>>>(w, x, y, n, k, bpu, units, nblocks, bias); break;
+    default: gemv_flat_kernel<8><<<grid, 256, 0, stream>>>(w, x, y, n, k, bpu, units, nblocks, bias); break;
     }
     return hipGetLastError();
 }

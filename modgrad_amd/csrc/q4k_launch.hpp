@@ -159,9 +159,10 @@ hipError_t dequant_launch(const uint8_t *q, int n_blocks, float *out, hipStream_
 hipError_t gemv_generic_launch(const uint8_t *w, const float *x, float *y, int n, int k,
                                hipStream_t stream);
 // Flat-stream layout with k % 32 == 0 (whole sub-blocks per row), w and x
-// 16-byte aligned; hipErrorNotSupported otherwise (then: generic).
+// 16-byte aligned; hipErrorNotSupported otherwise (then: generic). A bias (n
+// floats, or null) is added to the row sums.
 hipError_t gemv_flat_launch(const uint8_t *w, const float *x, float *y, int n, int k,
-                            hipStream_t stream);
+                            hipStream_t stream, const float *bias = nullptr);
 
 // Matrix-core GEMV for the row-aligned layout. Returns hipErrorNotSupported
 // when the shape or alignment does not fit it (caller then uses generic).

@@ -306,6 +306,19 @@ class kern:
                                               _stream_ptr(stream)), "matvec_q4k_ex")
 
     @staticmethod
+    def matvec_q4k_bias(w: int, x: int, bias: int, y: int, out_dim: int, k_elems: int,
+                        layout: int = _lib.LAYOUT_ROWS, stream=None) -> None:
+        """y = W x + bias: matvec_q4k_ex then residual_add (same bits), in one
+        launch where bias_fuses(k_elems, layout)."""
+        _chk(_lib.load().launch_matvec_q4k_bias_ex(w, x, bias, y, out_dim, k_elems, layout,
+                                                   _stream_ptr(stream)), "matvec_q4k_bias")
+
+    @staticmethod
+    def bias_fuses(k_elems: int, layout: int) -> bool:
+        """Whether matvec_q4k_bias is one kernel (else two)."""
+        return layout == _lib.LAYOUT_FLAT and k_elems % 32 == 0 and k_elems % 256 != 0
+
+    @staticmethod
     def batched_workspace_bytes(bpr: int, batch: int) -> int:
         return int(_lib.load().mgq_batched_workspace_bytes(bpr, batch))
 
@@ -764,12 +777,11 @@ class LinearResidentQuantized:
         With a HipBatch, every kernel queued here counts against it."""
         x_buf, out_buf = _hip_of(x_dev, "x"), _hip_of(out_dev, "out")
         self.ensure_resident(batch)
-        kern.matvec_q4k_ex(self.weight_q4k_dev.device_ptr(), x_buf.device_ptr(),
-                           out_buf.device_ptr(), self._out, self._in, _lib.LAYOUT_FLAT, stream)
+        kern.matvec_q4k_bias(self.weight_q4k_dev.device_ptr(), x_buf.device_ptr(),
+                             self.bias_dev.device_ptr(), out_buf.device_ptr(), self._out, self._in,
+                             _lib.LAYOUT_FLAT, stream)
         if batch is not None:
-            batch.note_dispatch()
-        kern.residual_add(out_buf.device_ptr(), self.bias_dev.device_ptr(), self._out, stream)
-        if batch is not None:
-            batch.note_dispatch()
+            for _ in range(1 if kern.bias_fuses(self._in, _lib.LAYOUT_FLAT) else 2):
+                batch.note_dispatch()
         if auto_evict:
             self.evict()
