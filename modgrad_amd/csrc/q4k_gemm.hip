@@ -25,6 +25,10 @@
 //     straight into LDS (global_load_lds, no registers), NBUF - 1 half blocks
 //     ahead. It issues no other vector memory operation, so its vmcnt waits
 //     are exact; the compute wavefronts' loads are waited for by the compiler.
+//   * The two wavefronts of a SIMD run a half block's dequantization and
+//     products in opposite orders (run), so that one's vector work falls under
+//     the other's matrix work: 3584 x 18944 at 512 tokens 105 -> 95 us, at 4096
+//     553 -> 508.
 //   * One barrier per half block. After the K loop the NWK partial tiles are
 //     added in LDS in a fixed order (the result does not depend on timing).
 // Splitting K inside the work-group is what fills the chip when there are few
@@ -201,12 +205,12 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
 #pragma unroll
     for (int i = 0; i < RT; ++i)
         woff[i] = (Off)(min(r0 + 16 * i + l16, n - 1) - rb) * (Off)row_bytes + 16u * q;
-    // header loads: a row a lane, 64 rows a load (RT == 1: a row on 4 lanes)
+    // header loads: a row a lane, 64 rows a load (RT == 1, 2: a row on 4, 2 lanes)
     constexpr int HD = (RT + 3) / 4;
     Off hoff[HD];
 #pragma unroll
     for (int k = 0; k < HD; ++k) {
-        const int row = RT == 1 ? l16 : min(64 * k + lane, 16 * RT - 1);
+        const int row = RT == 1 ? l16 : RT == 2 ? (lane & 31) : min(64 * k + lane, 16 * RT - 1);
         hoff[k] = (Off)(min(r0 + row, n - 1) - rb) * (Off)row_bytes;
     }
     u32x4 Wr[PD][2][RT], Hd[PD][HD];  // qs and headers of the next PD blocks
@@ -229,7 +233,9 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
 #pragma unroll
     for (int k = 0; k < HD; ++k) { er[k] = gemm::kNoExp; del[k] = 0; }
     uint8_t *stab = lds + L::OS + wave * (2 * L::ST);
-    const uint32_t mA = q < 2 ? 0x3F3F3F3Fu : 0x0F0F0F0Fu, mB = q < 2 ? 0u : 0x30303030u, qsh = 16u * (q & 1);
+    // (RT <= 2: the lane's sub-blocks are in the first or the second half)
+    const bool first4 = q < 2;
+    const uint32_t mA = first4 ? 0x3F3F3F3Fu : 0x0F0F0F0Fu, mB = first4 ? 0u : 0x30303030u, qsh = 16u * (q & 1);
     // the sub-block pair at bits o.. of sc and mn (even one, odd one: high
     // nibbles arrive as 16 q)
     auto pairs = [](float d, float d16, float nm, uint32_t sc, uint32_t mn, int o) __attribute__((always_inline)) {
@@ -253,10 +259,16 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
             any |= del[k];
             er[k] = e;
             const float d = ldexpf(dh, e + 4), d16 = ldexpf(dh, e), nm = -ldexpf(mh, e - 20);
-            if constexpr (RT == 1) {  // lane group q: sub-blocks 2q, 2q + 1
-                const uint32_t sc = (((q < 2 ? s0 : s2) & mA) | ((s0 >> 2) & mB)) >> qsh;
-                const uint32_t mn = (((q < 2 ? s1 : s2 >> 4) & mA) | ((s1 >> 2) & mB)) >> qsh;
-                *reinterpret_cast<u32x2 *>(stab + buf * L::ST + l16 * gemm::SROW + 8 * q) = pairs(d, d16, nm, sc, mn, 0);
+            if constexpr (RT <= 2) {
+                const uint32_t sc = ((first4 ? s0 : s2) & mA) | ((s0 >> 2) & mB);
+                const uint32_t mn = ((first4 ? s1 : s2 >> 4) & mA) | ((s1 >> 2) & mB);
+                if constexpr (RT == 1) {  // lane group q: sub-blocks 2q, 2q + 1
+                    *reinterpret_cast<u32x2 *>(stab + buf * L::ST + l16 * gemm::SROW + 8 * q) = pairs(d, d16, nm, sc >> qsh, mn >> qsh, 0);
+                } else {  // half-wavefront h: sub-blocks 4h .. 4h + 3
+                    u32x2 *dst = reinterpret_cast<u32x2 *>(stab + buf * L::ST + (lane & 31) * gemm::SROW + 16 * (lane >> 5));
+                    dst[0] = pairs(d, d16, nm, sc, mn, 0);
+                    dst[1] = pairs(d, d16, nm, sc, mn, 16);
+                }
             } else {
                 const int row = min(64 * k + lane, 16 * RT - 1);
                 u32x2 *dst = reinterpret_cast<u32x2 *>(stab + buf * L::ST + row * gemm::SROW);
@@ -282,24 +294,15 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
         for (int j = 0; j < TT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     const uint32_t chunk0 = (uint32_t)(8 * (q >> 1) + 2 * (q & 1));
     const uint8_t *abuf0 = lds + (uint32_t)kg * NBUF * L::SA + l16 * 256;
-    // half block H from token buffer `buf` and scale table `tab`
-    auto compute = [&](auto hc, auto uc, int buf, int tab) __attribute__((always_inline)) {
-        constexpr int H = decltype(hc)::value, U = decltype(uc)::value;
-        constexpr int SETS = TT <= 3 ? 4 : 2;  // slots whose token operands are in registers
-        half8 tb[SETS][TT];
-        auto read = [&](int s) __attribute__((always_inline)) {
-            const uint8_t *p = abuf0 + buf * L::SA + ((chunk0 + (s & 1) + 4 * (s >> 1)) ^ (uint32_t)l16) * 16;
-#pragma unroll
-            for (int j = 0; j < TT; ++j) tb[s % SETS][j] = *reinterpret_cast<const half8 *>(p + j * 4096);
-        };
-        u32x2 sp[RT];
+    u32x4 op[RT][4];  // W operands of a half block: slot (j, hi) at 2 hi + j
+    u32x2 sp[RT];
+    auto read_scales = [&](int H, int tab) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < RT; ++i)
             sp[i] = *reinterpret_cast<const u32x2 *>(stab + tab * L::ST + (16 * i + l16) * gemm::SROW + 16 * H + 8 * (q >> 1));
-#pragma unroll
-        for (int s = 0; s < SETS - (SETS == 4 ? 0 : 1); ++s) read(s);
-        __builtin_amdgcn_sched_barrier(0);
-        u32x4 op[RT][4];  // slot (j, hi) at 2 hi + j
+    };
+    auto dequant = [&](auto hc, auto uc) __attribute__((always_inline)) {
+        constexpr int H = decltype(hc)::value, U = decltype(uc)::value;
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
             const uint32_t sp0 = sp[i][0], sp1 = sp[i][1];
@@ -316,10 +319,24 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
                 op[i][2 + (u >> 1)][2 * (u & 1) + 1] = dqs2(p1, 0x00F000F0u, dh, nh);
             }
         }
+    };
+    constexpr int SETS = TT <= 3 ? 4 : 2;  // slots whose token operands are in registers
+    half8 tb[SETS][TT];
+    auto read = [&](int s, int buf) __attribute__((always_inline)) {
+        const uint8_t *p = abuf0 + buf * L::SA + ((chunk0 + (s & 1) + 4 * (s >> 1)) ^ (uint32_t)l16) * 16;
+#pragma unroll
+        for (int j = 0; j < TT; ++j) tb[s % SETS][j] = *reinterpret_cast<const half8 *>(p + j * 4096);
+    };
+    auto read_ahead = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < (SETS == 4 ? 4 : 1); ++s) read(s, buf);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto products = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             if constexpr (SETS == 2) {
-                if (s < 3) read(s + 1);
+                if (s < 3) read(s + 1, buf);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
@@ -346,53 +363,107 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
             for (int j = 0; j < TT; ++j) acc[i][j] *= f;
         }
     };
-    // Loads go out in one order, the prologue's included, so that every wait
-    // leaves the younger ones in flight: qs half 0 of block t, the header of
-    // t + 1, qs half 1 of t.
-    loadH(kg, H0{});
-    __builtin_amdgcn_sched_barrier(0);
-    decode(H0{}, 0, NWK == 1 || kg < bpr);
-    auto first = [&](auto uc) __attribute__((always_inline)) {
-        constexpr int U = decltype(uc)::value;
-        if constexpr (U < PD) {
-            loadW(kg + U * NWK, H0{}, uc);
+    // Two orders of the same work, one for the even and one for the odd
+    // wavefronts of each SIMD, so that one dequantizes while the other
+    // multiplies: (late = 0) a half block's dequantization, then its products;
+    // (late = 1) its products, then the next half block's dequantization. The
+    // next block's header is decoded in half 1 or half 0. Loads go out in one
+    // order, the prologue's included, so that every wait leaves the younger
+    // ones in flight.
+    auto run = [&](auto late) __attribute__((always_inline)) {
+        constexpr bool LATE = decltype(late)::value;
+        loadH(kg, H0{});
+        __builtin_amdgcn_sched_barrier(0);
+        decode(H0{}, 0, NWK == 1 || kg < bpr);
+        auto first = [&](auto uc) __attribute__((always_inline)) {
+            constexpr int U = decltype(uc)::value;
+            if constexpr (U < PD) {
+                loadW(kg + U * NWK, H0{}, uc);
+                __builtin_amdgcn_sched_barrier(0);
+                loadH(kg + (U + 1) * NWK, std::integral_constant<int, (U + 1) % PD>{});
+                __builtin_amdgcn_sched_barrier(0);
+                loadW(kg + U * NWK, H1{}, uc);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        first(H0{});
+        first(H1{});
+        if constexpr (LATE) {
+            read_scales(0, 0);
+            dequant(H0{}, H0{});
             __builtin_amdgcn_sched_barrier(0);
-            loadH(kg + (U + 1) * NWK, std::integral_constant<int, (U + 1) % PD>{});
-            __builtin_amdgcn_sched_barrier(0);
-            loadW(kg + U * NWK, H1{}, uc);
+            loadW(kg + PD * NWK, H0{}, H0{});
             __builtin_amdgcn_sched_barrier(0);
         }
+        lds_barrier();  // half block 0 is in LDS
+        auto block = [&](int t, auto uc) __attribute__((always_inline)) {
+            constexpr int U = decltype(uc)::value;
+            using N = std::integral_constant<int, (U + 1) % PD>;  // the next block's registers
+            const int b = kg + t * NWK, tab = t & 1;
+            const bool live = NWK == 1 || b < bpr;  // uniform
+            const bool on = NWK == 1 || b + NWK < bpr;
+            bool changed = false;
+            if constexpr (LATE) {
+                if (live) {
+                    read_ahead(buf);
+                    products(buf);
+                }
+                read_scales(1, tab);
+                changed = decode(N{}, tab ^ 1, on);
+                __builtin_amdgcn_sched_barrier(0);
+                loadH(b + (1 + PD) * NWK, N{});
+                dequant(H1{}, uc);
+                __builtin_amdgcn_sched_barrier(0);
+                loadW(b + PD * NWK, H1{}, uc);
+                __builtin_amdgcn_sched_barrier(0);
+                next_buf();
+                if (live) {
+                    read_ahead(buf);
+                    products(buf);
+                }
+                read_scales(0, tab ^ 1);
+                dequant(H0{}, N{});
+                __builtin_amdgcn_sched_barrier(0);
+                loadW(b + (1 + PD) * NWK, H0{}, N{});
+                __builtin_amdgcn_sched_barrier(0);
+            } else {
+                if (live) {
+                    read_scales(0, tab);
+                    read_ahead(buf);
+                    dequant(H0{}, uc);
+                    products(buf);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                loadW(b + PD * NWK, H0{}, uc);
+                __builtin_amdgcn_sched_barrier(0);
+                next_buf();
+                changed = decode(N{}, tab ^ 1, on);
+                __builtin_amdgcn_sched_barrier(0);
+                loadH(b + (1 + PD) * NWK, N{});
+                if (live) {
+                    read_scales(1, tab);
+                    read_ahead(buf);
+                    dequant(H1{}, uc);
+                    products(buf);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                loadW(b + PD * NWK, H1{}, uc);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (changed) rescale();  // rare
+            next_buf();
+        };
+        static_assert(PD == 1 || PD == 2, "blocks of W in registers");
+        for (int t = 0; t < NB; t += PD) {
+            block(t, H0{});
+            if constexpr (PD == 2)
+                if (t + 1 < NB) block(t + 1, H1{});
+        }
     };
-    first(H0{});
-    first(H1{});
-    lds_barrier();  // half block 0 is in LDS
-    auto block = [&](int t, auto uc) __attribute__((always_inline)) {
-        constexpr int U = decltype(uc)::value;
-        using N = std::integral_constant<int, (U + 1) % PD>;  // the next block's header
-        const int b = kg + t * NWK;
-        const bool live = NWK == 1 || b < bpr;  // uniform
-        if (live) compute(H0{}, uc, buf, t & 1);
-        __builtin_amdgcn_sched_barrier(0);
-        loadW(b + PD * NWK, H0{}, uc);
-        __builtin_amdgcn_sched_barrier(0);
-        next_buf();
-        // the next block's scales, in the other table
-        const bool changed = decode(N{}, (t + 1) & 1, NWK == 1 || b + NWK < bpr);
-        __builtin_amdgcn_sched_barrier(0);
-        loadH(b + (1 + PD) * NWK, N{});
-        if (live) compute(H1{}, uc, buf, t & 1);
-        __builtin_amdgcn_sched_barrier(0);
-        loadW(b + PD * NWK, H1{}, uc);
-        __builtin_amdgcn_sched_barrier(0);
-        if (changed) rescale();  // rare
-        next_buf();
-    };
-    static_assert(PD == 1 || PD == 2, "blocks of W in registers");
-    for (int t = 0; t < NB; t += PD) {
-        block(t, H0{});
-        if constexpr (PD == 2)
-            if (t + 1 < NB) block(t + 1, H1{});
-    }
+    // (336 x 128's accumulators leave no registers for the second order)
+    constexpr bool PAIRED = L::NC > 4 && RT * TT <= 16;
+    if (PAIRED && (wave & 4)) run(std::integral_constant<bool, PAIRED>{});
+    else run(std::false_type{});
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
         const f32x4 f = row_pow2(er, i, 20, -1);
@@ -461,7 +532,7 @@ static hipError_t launch_tile(const uint8_t *w, const uint16_t *a, float *c, int
 // its K share, with every CU holding one; a call takes as many rounds of that
 // as its tiles fill (rounds of all CUs, the last one counted whole). Fitted to
 // 438 shapes (N 576-37888, K 1536-18944, M 17-2048): the predicted best shape
-// is within 0.8 % of the measured best on average, 20 % at worst. W's prefetch
+// is within 0.4 % of the measured best on average, 17 % at worst. W's prefetch
 // is two blocks where the registers allow it without losing a wavefront.
 struct GemmTile {
     int bn, bm, nwk;
@@ -471,20 +542,20 @@ struct GemmTile {
 #define MGQ_TILE(RT, TT, NWN, NWK, NBUF, PD, FIXED, BLOCK) \
     {16 * RT * NWN, 16 * TT, NWK, FIXED, BLOCK, launch_tile<RT, TT, NWN, NWK, NBUF, PD, uint32_t>}
 static const GemmTile kTiles[] = {
-    MGQ_TILE(1, 1, 2, 4, 4, 2, 1.7f, 1.06f),   //  32 x  16
-    MGQ_TILE(1, 2, 2, 4, 4, 1, 2.2f, 1.36f),   //  32 x  32
-    MGQ_TILE(1, 3, 2, 4, 3, 1, 2.4f, 1.63f),   //  32 x  48
-    MGQ_TILE(1, 3, 4, 2, 3, 2, 3.1f, 1.20f),   //  64 x  48
-    MGQ_TILE(2, 5, 2, 2, 3, 2, 4.1f, 1.50f),   //  64 x  80
-    MGQ_TILE(2, 3, 4, 2, 4, 1, 3.9f, 1.97f),   // 128 x  48
-    MGQ_TILE(2, 4, 4, 2, 3, 1, 4.3f, 2.07f),   // 128 x  64
-    MGQ_TILE(2, 5, 4, 2, 3, 1, 5.0f, 2.27f),   // 128 x  80
-    MGQ_TILE(1, 3, 10, 1, 4, 2, 3.6f, 1.29f),  // 160 x  48
-    MGQ_TILE(2, 3, 5, 2, 4, 1, 4.6f, 2.49f),   // 160 x  48, K in two shares
-    MGQ_TILE(2, 5, 5, 2, 3, 1, 6.0f, 2.83f),   // 160 x  80
-    MGQ_TILE(2, 8, 7, 1, 2, 1, 5.9f, 2.77f),   // 224 x 128
-    MGQ_TILE(3, 5, 7, 1, 3, 1, 6.0f, 2.76f),   // 336 x  80
-    MGQ_TILE(3, 8, 7, 1, 2, 1, 7.7f, 3.68f),   // 336 x 128
+    MGQ_TILE(1, 1, 2, 4, 4, 2, 1.8f, 1.08f),   //  32 x  16
+    MGQ_TILE(1, 2, 2, 4, 4, 1, 2.2f, 1.43f),   //  32 x  32
+    MGQ_TILE(1, 3, 2, 4, 3, 1, 2.4f, 1.68f),   //  32 x  48
+    MGQ_TILE(1, 3, 4, 2, 3, 2, 2.7f, 1.31f),   //  64 x  48
+    MGQ_TILE(2, 5, 2, 2, 3, 2, 3.8f, 1.48f),   //  64 x  80
+    MGQ_TILE(2, 3, 4, 2, 4, 1, 3.7f, 1.92f),   // 128 x  48
+    MGQ_TILE(2, 4, 4, 2, 3, 1, 4.3f, 2.11f),   // 128 x  64
+    MGQ_TILE(2, 5, 4, 2, 3, 1, 5.1f, 2.32f),   // 128 x  80
+    MGQ_TILE(1, 3, 10, 1, 4, 2, 3.8f, 1.30f),  // 160 x  48
+    MGQ_TILE(2, 3, 5, 2, 4, 1, 4.4f, 2.31f),   // 160 x  48, K in two shares
+    MGQ_TILE(2, 5, 5, 2, 3, 1, 5.9f, 2.77f),   // 160 x  80
+    MGQ_TILE(2, 8, 7, 1, 2, 1, 6.4f, 2.80f),   // 224 x 128
+    MGQ_TILE(3, 5, 7, 1, 3, 1, 6.0f, 2.70f),   // 336 x  80
+    MGQ_TILE(3, 8, 7, 1, 2, 1, 7.7f, 3.69f),   // 336 x 128
 };
 #undef MGQ_TILE
 // Rows so long that a tile's offsets pass 32 bits (K above ~16 million).

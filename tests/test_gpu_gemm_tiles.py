@@ -62,8 +62,8 @@ def check(L, orc, n, bpr, m, woff=0, aoff=0, coff=0):
     (20479, 1, 17), (30001, 3, 47),                               # 160 x 48
     (37888, 26, 33),                                              # 160 x 48, two K shares
     (20479, 2, 127), (20479, 3, 97),                              # 160 x 80
-    (42001, 1, 5), (42001, 3, 127),                               # 224 x 128
-    (60001, 2, 1), (85007, 3, 79),                                # 336 x 80
+    (56001, 4, 100), (7001, 4, 1021),                             # 224 x 128
+    (60001, 2, 1), (85007, 3, 79), (42001, 1, 5), (42001, 3, 127),  # 336 x 80
     (30001, 1, 161), (85007, 2, 81), (60001, 3, 127)])            # 336 x 128
 def test_gemm_tile_shapes(L, orc, n, bpr, m):
     note(f"gemm tiles n={n} bpr={bpr} m={m}")
