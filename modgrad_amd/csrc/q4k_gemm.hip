@@ -2,8 +2,8 @@
 //   C[m][r] = sum_k dequant(W)[r][k] * A[m][k],  A f16 [M][K], C f32 [M][N].
 // No counterpart in the reference (its prefill is a per-token GEMV loop,
 // crates/modgrad-gemma/examples/gemma4_rocm.rs:26-34); each weight is the
-// canonical dequantized value (gguf.rs:364-404) times a per-row power of two
-// 2^(e-20) that keeps it inside f16's range, with d*sc and dmin*m (times their
+// canonical dequantized value (gguf.rs:364-404) times a power of two 2^(e-20)
+// that keeps it inside f16's normal range, with d*sc and dmin*m (times their
 // powers of two) rounded to f16 and the weight computed and rounded once in
 // f16; C is scaled back exactly.
 //
@@ -44,22 +44,28 @@
 // chunk ^ (token % 16): the reads have no bank conflicts (counted: 0), and
 // the loader applies the swizzle to the addresses it reads from.
 //
-// Dequantization. A nibble masked in place is the f16 subnormal q * 2^-24 (or
-// 16 q * 2^-24), exact; one v_pk_fma_f16 with the sub-block pair
-// (d*sc*2^(e+4), -dmin*m*2^(e-20)) gives two weights * 2^(e-20), rounded
-// once: 2.5 VALU per pair with the byte permutes. Each lane decodes one row's
-// block header (a row on four lanes, a quarter each, when RT == 1) into 8
-// such pairs in a wave-private LDS table, one block ahead.
+// Dequantization. A nibble in bits 4..7 of an f16 is the subnormal q * 2^-20,
+// exact (low nibbles are shifted there, a dword at a time); one v_pk_fma_f16
+// with the sub-block pair (d*sc*2^e, -dmin*m*2^(e-20)) gives two weights *
+// 2^(e-20), rounded once: 2.75 VALU per pair with the byte permutes (low
+// nibbles left in bits 0..3 would save a shift per eight weights and cost four
+// binades of the weights' range). Each lane decodes one row's block header (a
+// row on four lanes, a quarter each, when RT == 1) into 8 such pairs in a
+// wave-private LDS table, one block ahead.
 //
-// Range. Each W row carries a running power-of-two exponent e. Any e at or
-// below tight = 15 - exponent(945|d| + 63|dmin|) of a block keeps its
-// |weight| * 2^e below 2^15. A row starts at tight - kRangeHeadroom of its
-// first nonzero block and keeps e while the later blocks' tight stays at or
-// above it; a block that overruns it lowers e to its tight - kRangeHeadroom,
-// and the wavefront multiplies its sums so far by 2^(e_new - e_old) (exact)
-// before that block's products. |d*sc| * 2^(e+4) < 2^15 * 63*16/945 stays
-// below the f16 maximum, and weights above 2^-(9 - kRangeHeadroom) of the
-// largest seen so far stay normal f16. C is multiplied by 2^(20-e) at the end.
+// Range. Each W row carries a running power-of-two exponent e. A block's
+// `tight` is the largest e that keeps its 63|d| * 2^e and 63|dmin| * 2^(e-19)
+// below 2^16, so that neither the multipliers nor the weights pass f16's
+// maximum. A row keeps e while tight - 2 kRangeHeadroom <= e <= tight; a block
+// outside that (the first nonzero one always is) sets e to its
+// tight - kRangeHeadroom, up or down, and the wavefront multiplies its sums so
+// far by 2^(e_new - e_old) (exact) before that block's products. A block's
+// largest multiplier is then 2^9 .. 2^16 and its d*sc*q * 2^(e-20) reach
+// 2^-8 .. 2^0: every sub-block, 2^6 below its block's largest or not, is held
+// in normal f16 numbers but for what a block's largest weights round away.
+// Sums in f32 do not overflow: a weight is below 2^15 in its own e, an
+// activation below 2^16, and e (-10 .. 53 over all finite headers) rises by 63
+// at most. C is multiplied by 2^(20-e) at the end.
 #include "q4k_device.hpp"
 #include "q4k_launch.hpp"
 
@@ -69,17 +75,18 @@ namespace mgq {
 
 namespace gemm {
 constexpr int NXCD = 8;             // XCDs the hardware deals work-groups across, round robin
-constexpr int kRangeHeadroom = 4;
-constexpr int kNoExp = 100;         // e of a row with no nonzero block yet (tight <= 34)
+constexpr int kRangeHeadroom = 3;   // blocks 2^3 either way of the first: no rescale
+constexpr int kNoExp = 100;         // e of a row with no nonzero block yet (tight <= 53)
 constexpr int SROW = 40;            // bytes per scale-table row (32 + pad: conflict-free b64 reads)
 constexpr int GROUP_M = 8;          // token tiles that share an XCD's W tiles
 }  // namespace gemm
 
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 
-// Two weights (bytes 0 and 2 of v, nibble selected by mask) as an f16 pair.
-__device__ __forceinline__ uint32_t dqs2(uint32_t v, uint32_t mask, h2_t d1, h2_t nm1) {
-    const h2_t q = __builtin_bit_cast(h2_t, v & mask);
+// Two weights from the quants 16 q in two bytes of v (pick: v_perm selector)
+// as an f16 pair.
+__device__ __forceinline__ uint32_t dqs2(uint32_t v, uint32_t pick, h2_t d1, h2_t nm1) {
+    const h2_t q = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(v, v, pick));
     return __builtin_bit_cast(uint32_t, q * d1 + nm1);
 }
 
@@ -236,11 +243,10 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
     // (RT <= 2: the lane's sub-blocks are in the first or the second half)
     const bool first4 = q < 2;
     const uint32_t mA = first4 ? 0x3F3F3F3Fu : 0x0F0F0F0Fu, mB = first4 ? 0u : 0x30303030u, qsh = 16u * (q & 1);
-    // the sub-block pair at bits o.. of sc and mn (even one, odd one: high
-    // nibbles arrive as 16 q)
-    auto pairs = [](float d, float d16, float nm, uint32_t sc, uint32_t mn, int o) __attribute__((always_inline)) {
+    // the sub-block pair at bits o.. of sc and mn (even one, odd one)
+    auto pairs = [](float d, float nm, uint32_t sc, uint32_t mn, int o) __attribute__((always_inline)) {
         const h2_t lo = {(_Float16)(d * (float)((sc >> o) & 0xFFu)), (_Float16)(nm * (float)((mn >> o) & 0xFFu))};
-        const h2_t hi = {(_Float16)(d16 * (float)((sc >> (o + 8)) & 0xFFu)),
+        const h2_t hi = {(_Float16)(d * (float)((sc >> (o + 8)) & 0xFFu)),
                          (_Float16)(nm * (float)((mn >> (o + 8)) & 0xFFu))};
         return u32x2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
     };
@@ -251,30 +257,32 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
         for (int k = 0; k < HD; ++k) {
             const uint32_t h0 = Hd[U][k][0], s0 = Hd[U][k][1], s1 = Hd[U][k][2], s2 = Hd[U][k][3];
             const float dh = half_bits_finite(h0), mh = half_bits_finite(h0 >> 16);
-            // 15 - exponent of the bound (zero or a normal number: d is an f16)
-            const float bound = fabsf(dh) * 945.0f + fabsf(mh) * 63.0f;
-            const int tight = 15 + 126 - (int)(__builtin_bit_cast(uint32_t, bound) >> 23);
-            const int e = (on && tight < er[k]) ? tight - gemm::kRangeHeadroom : er[k];
+            // 15 - exponent of the bound (a normal number, or zero and then
+            // 142; 64.1: f16 rounds below 65504)
+            const float bound = fabsf(dh) * 64.1f + fabsf(mh) * (63.0f / 524288.0f);
+            const int tight = 15 + 127 - (int)(__builtin_bit_cast(uint32_t, bound) >> 23);
+            const bool out = tight < er[k] || (tight > er[k] + 2 * gemm::kRangeHeadroom && tight < gemm::kNoExp);
+            const int e = (on && out) ? tight - gemm::kRangeHeadroom : er[k];
             del[k] = e - er[k];
             any |= del[k];
             er[k] = e;
-            const float d = ldexpf(dh, e + 4), d16 = ldexpf(dh, e), nm = -ldexpf(mh, e - 20);
+            const float d = ldexpf(dh, e), nm = -ldexpf(mh, e - 20);
             if constexpr (RT <= 2) {
                 const uint32_t sc = ((first4 ? s0 : s2) & mA) | ((s0 >> 2) & mB);
                 const uint32_t mn = ((first4 ? s1 : s2 >> 4) & mA) | ((s1 >> 2) & mB);
                 if constexpr (RT == 1) {  // lane group q: sub-blocks 2q, 2q + 1
-                    *reinterpret_cast<u32x2 *>(stab + buf * L::ST + l16 * gemm::SROW + 8 * q) = pairs(d, d16, nm, sc >> qsh, mn >> qsh, 0);
+                    *reinterpret_cast<u32x2 *>(stab + buf * L::ST + l16 * gemm::SROW + 8 * q) = pairs(d, nm, sc >> qsh, mn >> qsh, 0);
                 } else {  // half-wavefront h: sub-blocks 4h .. 4h + 3
                     u32x2 *dst = reinterpret_cast<u32x2 *>(stab + buf * L::ST + (lane & 31) * gemm::SROW + 16 * (lane >> 5));
-                    dst[0] = pairs(d, d16, nm, sc, mn, 0);
-                    dst[1] = pairs(d, d16, nm, sc, mn, 16);
+                    dst[0] = pairs(d, nm, sc, mn, 0);
+                    dst[1] = pairs(d, nm, sc, mn, 16);
                 }
             } else {
                 const int row = min(64 * k + lane, 16 * RT - 1);
                 u32x2 *dst = reinterpret_cast<u32x2 *>(stab + buf * L::ST + row * gemm::SROW);
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    dst[j] = pairs(d, d16, nm, scales4(j >> 1, s0, s2), mins4(j >> 1, s1, s2), 16 * (j & 1));
+                    dst[j] = pairs(d, nm, scales4(j >> 1, s0, s2), mins4(j >> 1, s1, s2), 16 * (j & 1));
             }
         }
         return __any(any != 0);
@@ -310,13 +318,12 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
             const h2_t dl = {sl[0], sl[0]}, nl = {sl[1], sl[1]}, dh = {sh[0], sh[0]}, nh = {sh[1], sh[1]};
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const uint32_t v = Wr[U][H][i][u];
-                const uint32_t p0 = __builtin_amdgcn_perm(v, v, 0x0C010C00u);  // bytes 0, 1 -> 0, 2
-                const uint32_t p1 = __builtin_amdgcn_perm(v, v, 0x0C030C02u);  // bytes 2, 3 -> 0, 2
-                op[i][u >> 1][2 * (u & 1)] = dqs2(p0, 0x000F000Fu, dl, nl);
-                op[i][u >> 1][2 * (u & 1) + 1] = dqs2(p1, 0x000F000Fu, dl, nl);
-                op[i][2 + (u >> 1)][2 * (u & 1)] = dqs2(p0, 0x00F000F0u, dh, nh);
-                op[i][2 + (u >> 1)][2 * (u & 1) + 1] = dqs2(p1, 0x00F000F0u, dh, nh);
+                const uint32_t v = Wr[U][H][i][u], lo = (v << 4) & 0xF0F0F0F0u, hi = v & 0xF0F0F0F0u;
+                constexpr uint32_t B01 = 0x0C010C00u, B23 = 0x0C030C02u;  // bytes -> 0, 2
+                op[i][u >> 1][2 * (u & 1)] = dqs2(lo, B01, dl, nl);
+                op[i][u >> 1][2 * (u & 1) + 1] = dqs2(lo, B23, dl, nl);
+                op[i][2 + (u >> 1)][2 * (u & 1)] = dqs2(hi, B01, dh, nh);
+                op[i][2 + (u >> 1)][2 * (u & 1) + 1] = dqs2(hi, B23, dh, nh);
             }
         }
     };
