@@ -173,29 +173,66 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
             const int t = 4 * i + q;
             aoff[i] = (Off)min(t, m_tokens - 1 - m0) * (Off)pitch + 16u * (l16 ^ (t & 15));
         }
-        const bool direct = ((uintptr_t)a & 15u) == 0;  // else through registers
-        auto copy = [&](int s) __attribute__((always_inline)) {
-            const uint8_t *src = abase + (size_t)blk(kg + (s >> 1) * NWK) * (kBlockElems * 2) + 256 * (s & 1);
-            const uint32_t dst = buf0 + (uint32_t)(s % NBUF) * L::SA;
-            if (direct) {
-#pragma unroll
-                for (int i = 0; i < L::IPS; ++i) lds_copy16(lds0 + dst + 1024u * i, src, aoff[i]);
-            } else {
-#pragma unroll 2
-                for (int i = 0; i < L::IPS; ++i)
-                    *reinterpret_cast<u32x4 *>(lds + dst + 1024u * i + 16 * lane) = ld_u32x4(src + aoff[i]);
-            }
+        auto half_at = [&](int s) __attribute__((always_inline)) {
+            return abase + (size_t)blk(kg + (s >> 1) * NWK) * (kBlockElems * 2) + 256 * (s & 1);
         };
+        auto buf_at = [&](int s) __attribute__((always_inline)) { return buf0 + (uint32_t)(s % NBUF) * L::SA; };
+        if (((uintptr_t)a & 15u) == 0) {
+            auto copy = [&](int s) __attribute__((always_inline)) {
+                const uint8_t *src = half_at(s);
+                const uint32_t dst = lds0 + buf_at(s);
 #pragma unroll
-        for (int s = 0; s < NBUF; ++s) copy(s);
-        vm_wait<(NBUF - 1) * L::IPS>();  // half block 0 has landed
-        lds_barrier();
-        for (int s = 0; s < 2 * NB; ++s) {
-            vm_wait<(NBUF - 2) * L::IPS>();  // half block s + 1 has landed
-            lds_barrier();                   // half block s has been read
-            copy(s + NBUF);
+                for (int i = 0; i < L::IPS; ++i) lds_copy16(dst + 1024u * i, src, aoff[i]);
+            };
+#pragma unroll
+            for (int s = 0; s < NBUF; ++s) copy(s);
+            vm_wait<(NBUF - 1) * L::IPS>();  // half block 0 has landed
+            lds_barrier();
+            for (int s = 0; s < 2 * NB; ++s) {
+                vm_wait<(NBUF - 2) * L::IPS>();  // half block s + 1 has landed
+                lds_barrier();                   // half block s has been read
+                copy(s + NBUF);
+            }
+            vm_wait<0>();
+        } else {
+            // A off 16 bytes: through registers, half block s in set s % D, D
+            // half blocks in flight (18944 x 3584 at 512 tokens: 321 us with
+            // two pieces in flight -> 78, aligned 78-82)
+            constexpr int D = L::IPS <= 8 ? 4 : L::IPS <= 16 ? 2 : 1;
+            u32x4 R[D][L::IPS];
+            auto fetch = [&](int s, int set) __attribute__((always_inline)) {
+                const uint8_t *src = half_at(s);
+#pragma unroll
+                for (int i = 0; i < L::IPS; ++i) {
+                    Off off = aoff[i];
+                    asm("" : "+v"(off));  // not widened to a register pair ahead of the loop
+                    R[set][i] = ld_u32x4(src + off);
+                }
+            };
+            auto put = [&](int s, int set) __attribute__((always_inline)) {
+                uint8_t *dst = lds + buf_at(s) + 16 * lane;
+#pragma unroll
+                for (int i = 0; i < L::IPS; ++i) *reinterpret_cast<u32x4 *>(dst + 1024u * i) = R[set][i];
+                __builtin_amdgcn_sched_barrier(0);  // the set's next loads take its registers
+            };
+#pragma unroll
+            for (int s = 0; s < D; ++s) fetch(s, s);
+            put(0, 0);
+            fetch(D, 0);
+            lds_barrier();
+            for (int s0 = 0; s0 < 2 * NB; s0 += D) {
+#pragma unroll
+                for (int u = 0; u < D; ++u) {
+                    const int s = s0 + u;
+                    if (s >= 2 * NB) break;  // uniform
+                    // into the buffer of half block s + 1 - NBUF, read before
+                    // the barrier that half block s began behind
+                    put(s + 1, (u + 1) % D);
+                    fetch(s + 1 + D, (u + 1) % D);
+                    lds_barrier();  // half block s has been read
+                }
+            }
         }
-        vm_wait<0>();
         if constexpr (NWK > 1) {  // the partial tiles' two barriers
             lds_barrier();
             lds_barrier();

@@ -118,3 +118,32 @@ def test_gemm_first_call_in_a_graph():
     r = subprocess.run([sys.executable, "-c", CAPTURE, ROOT], capture_output=True, text=True,
                        timeout=110)
     assert r.returncode == 0 and "replays equal" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
+
+
+# A off 16 bytes takes the loader's registers: within twice the time of the
+# direct copies (median of 9; 0.95 to 1.35 measured, and 2.6 to 4.5 when the
+# loader waited for two pieces at a time)
+@pytest.mark.parametrize("n,bpr,m", [(3584, 14, 160), (4608, 14, 512), (18944, 14, 512), (2304, 26, 2048)])
+def test_gemm_unaligned_activations_time(L, n, bpr, m):
+    import torch
+    note(f"gemm time n={n} bpr={bpr} m={m}, A at +0 and +2")
+    wt = dev(random_q4k_bytes(np.random.default_rng(1), n * bpr))
+    at = dev(np.random.default_rng(2).standard_normal(m * bpr * 256 + 8).astype(np.float16))
+    ct = empty_f32(m * n)
+
+    def us(off, reps=20):
+        t = []
+        for _ in range(9):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            for _ in range(reps):
+                _lib.check("gemm", L.launch_gemm_q4k_f16(ptr(wt), ptr(at) + off, ptr(ct), n, bpr, m, None))
+            e[1].record()
+            e[1].synchronize()
+            t.append(e[0].elapsed_time(e[1]) / reps * 1e3)
+        return float(np.median(t))
+
+    us(0, 3), us(2, 3)
+    aligned, off2 = us(0), us(2)
+    print(f"aligned {aligned:.1f} us, at +2 {off2:.1f} us", flush=True)
+    assert off2 <= 2.0 * aligned
