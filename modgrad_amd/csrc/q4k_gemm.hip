@@ -24,7 +24,8 @@
 //   * The loader copies the tokens' 128-value half blocks from memory
 //     straight into LDS (global_load_lds, no registers), NBUF - 1 half blocks
 //     ahead. It issues no other vector memory operation, so its vmcnt waits
-//     are exact; the compute wavefronts' loads are waited for by the compiler.
+//     are exact (a register spilled around them would make them stricter);
+//     the compute wavefronts' loads are waited for by the compiler.
 //   * The two wavefronts of a SIMD run a half block's dequantization and
 //     products in opposite orders (run), so that one's vector work falls under
 //     the other's matrix work: 3584 x 18944 at 512 tokens 105 -> 95 us, at 4096
@@ -90,17 +91,14 @@ __device__ __forceinline__ uint32_t dqs2(uint32_t v, uint32_t pick, h2_t d1, h2_
     return __builtin_bit_cast(uint32_t, q * d1 + nm1);
 }
 
-// Copies 16 bytes per lane from base + off to LDS bytes dst + 16 * lane (M0
-// takes one wait state before the copy reads it). Asm, so that the compiler
-// neither counts it in vmcnt nor waits for it before unrelated LDS reads;
-// the caller waits with vm_wait.
-__device__ __forceinline__ void lds_copy16(uint32_t dst, const uint8_t *base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base)
-                 : "memory");
-}
-__device__ __forceinline__ void lds_copy16(uint32_t dst, const uint8_t *base, uint64_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(base + off)
-                 : "memory");
+// Copies 16 bytes per lane from base + off to LDS bytes dst + 16 * lane (no
+// registers; the compiler sets M0). The caller waits with vm_wait.
+template <class Off>
+__device__ __forceinline__ void lds_copy16(uint8_t *dst, const uint8_t *base, Off &off) {
+    asm("" : "+s"(base));  // base and offset kept apart: no address arithmetic per copy
+    asm("" : "+v"(off));
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(base + off),
+                                     (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
 }
 // At most N of this wavefront's vector memory operations still in flight.
 template <int N>
@@ -163,7 +161,6 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
         // (token 4i + lane / 16) fetches the chunk that belongs at its place.
         // Tokens past m_tokens re-read the last one (never stored).
         const int kg = wave - L::NC;
-        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
         const uint32_t buf0 = (uint32_t)kg * NBUF * L::SA;
         const size_t pitch = (size_t)bpr * kBlockElems * 2;
         const uint8_t *abase = reinterpret_cast<const uint8_t *>(a) + (size_t)m0 * pitch;
@@ -180,7 +177,7 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
         if (((uintptr_t)a & 15u) == 0) {
             auto copy = [&](int s) __attribute__((always_inline)) {
                 const uint8_t *src = half_at(s);
-                const uint32_t dst = lds0 + buf_at(s);
+                uint8_t *dst = lds + buf_at(s);
 #pragma unroll
                 for (int i = 0; i < L::IPS; ++i) lds_copy16(dst + 1024u * i, src, aoff[i]);
             };
@@ -204,9 +201,8 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
                 const uint8_t *src = half_at(s);
 #pragma unroll
                 for (int i = 0; i < L::IPS; ++i) {
-                    Off off = aoff[i];
-                    asm("" : "+v"(off));  // not widened to a register pair ahead of the loop
-                    R[set][i] = ld_u32x4(src + off);
+                    asm("" : "+v"(aoff[i]));  // not widened to a register pair
+                    R[set][i] = ld_u32x4(src + aoff[i]);
                 }
             };
             auto put = [&](int s, int set) __attribute__((always_inline)) {
@@ -433,6 +429,7 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
         first(H0{});
         first(H1{});
         if constexpr (LATE) {
+            asm volatile("" ::: "memory");  // other lanes' table entries: read after decode's stores
             read_scales(0, 0);
             dequant(H0{}, H0{});
             __builtin_amdgcn_sched_barrier(0);
