@@ -559,7 +559,8 @@ static hipError_t launch_tile(const uint8_t *w, const uint16_t *a, float *c, int
                               hipStream_t stream) {
     using L = GemmLayout<RT, TT, NWN, NWK, NBUF>;
     auto kern = gemm_q4k_f16_kernel<RT, TT, NWN, NWK, NBUF, PD, Off>;
-    const hipError_t attr = allow_full_lds_by_addr((const void *)kern);
+    static std::atomic<int> lds_state[64];  // one per instance: no lock on a launch
+    const hipError_t attr = allow_full_lds((const void *)kern, lds_state);
     if (attr != hipSuccess || w == nullptr) return attr;  // w null: attribute only (gemm_prepare)
     const int tn = (n + L::BN - 1) / L::BN, tm = (m_tokens + L::BM - 1) / L::BM;
     const long ntiles = (long)tn * tm;
