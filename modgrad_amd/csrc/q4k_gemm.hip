@@ -91,6 +91,23 @@ __device__ __forceinline__ uint32_t dqs2(uint32_t v, uint32_t pick, h2_t d1, h2_
     return __builtin_bit_cast(uint32_t, q * d1 + nm1);
 }
 
+// Byte B of v as a float (written out: the compiler, knowing that the byte has
+// six bits, takes two operations).
+template <int B>
+__device__ __forceinline__ float ubyte_f32(uint32_t v) {
+    float f;
+    if constexpr (B == 0) asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(f) : "v"(v));
+    if constexpr (B == 1) asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(f) : "v"(v));
+    if constexpr (B == 2) asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(f) : "v"(v));
+    if constexpr (B == 3) asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(f) : "v"(v));
+    return f;
+}
+// half_bits_finite in one operation less.
+__device__ __forceinline__ float finite_half(uint32_t h) {
+    const float f = (float)__builtin_bit_cast(_Float16, (uint16_t)h);
+    return fabsf(f) < 65536.0f ? f : 0.0f;  // infinities and NaN -> 0
+}
+
 // Copies 16 bytes per lane from base + off to LDS bytes dst + 16 * lane (no
 // registers; the compiler sets M0). The caller waits with vm_wait.
 template <class Off>
@@ -276,49 +293,54 @@ __global__ __launch_bounds__(64 * (NWN + 1) * NWK) void gemm_q4k_f16_kernel(
     // (RT <= 2: the lane's sub-blocks are in the first or the second half)
     const bool first4 = q < 2;
     const uint32_t mA = first4 ? 0x3F3F3F3Fu : 0x0F0F0F0Fu, mB = first4 ? 0u : 0x30303030u, qsh = 16u * (q & 1);
-    // the sub-block pair at bits o.. of sc and mn (even one, odd one)
-    auto pairs = [](float d, float nm, uint32_t sc, uint32_t mn, int o) __attribute__((always_inline)) {
-        const h2_t lo = {(_Float16)(d * (float)((sc >> o) & 0xFFu)), (_Float16)(nm * (float)((mn >> o) & 0xFFu))};
-        const h2_t hi = {(_Float16)(d * (float)((sc >> (o + 8)) & 0xFFu)),
-                         (_Float16)(nm * (float)((mn >> (o + 8)) & 0xFFu))};
+    // the sub-block pair in bytes B, B + 1 of sc and mn (even one, odd one)
+    auto pairs = [](float d, float nm, uint32_t sc, uint32_t mn, auto bc) __attribute__((always_inline)) {
+        constexpr int B = decltype(bc)::value;
+        const h2_t lo = {(_Float16)(d * ubyte_f32<B>(sc)), (_Float16)(nm * ubyte_f32<B>(mn))};
+        const h2_t hi = {(_Float16)(d * ubyte_f32<B + 1>(sc)), (_Float16)(nm * ubyte_f32<B + 1>(mn))};
         return u32x2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
     };
+    using B0 = std::integral_constant<int, 0>;
+    using B2 = std::integral_constant<int, 2>;
     auto decode = [&](auto uc, int buf, bool on) __attribute__((always_inline)) -> bool {
         constexpr int U = decltype(uc)::value;
-        int any = 0;
+        bool any = false;
 #pragma unroll
         for (int k = 0; k < HD; ++k) {
             const uint32_t h0 = Hd[U][k][0], s0 = Hd[U][k][1], s1 = Hd[U][k][2], s2 = Hd[U][k][3];
-            const float dh = half_bits_finite(h0), mh = half_bits_finite(h0 >> 16);
-            // 15 - exponent of the bound (a normal number, or zero and then
-            // 142; 64.1: f16 rounds below 65504)
+            const float dh = finite_half(h0), mh = finite_half(h0 >> 16);
+            // 15 - exponent of the bound (a normal number, or zero; 64.1: f16
+            // rounds below 65504)
             const float bound = fabsf(dh) * 64.1f + fabsf(mh) * (63.0f / 524288.0f);
             const int tight = 15 + 127 - (int)(__builtin_bit_cast(uint32_t, bound) >> 23);
-            const bool out = tight < er[k] || (tight > er[k] + 2 * gemm::kRangeHeadroom && tight < gemm::kNoExp);
-            const int e = (on && out) ? tight - gemm::kRangeHeadroom : er[k];
+            const bool out = on && bound > 0.0f && (uint32_t)(tight - er[k]) > 2 * gemm::kRangeHeadroom;
+            const int e = out ? tight - gemm::kRangeHeadroom : er[k];
             del[k] = e - er[k];
-            any |= del[k];
+            any |= out;
             er[k] = e;
             const float d = ldexpf(dh, e), nm = -ldexpf(mh, e - 20);
             if constexpr (RT <= 2) {
                 const uint32_t sc = ((first4 ? s0 : s2) & mA) | ((s0 >> 2) & mB);
                 const uint32_t mn = ((first4 ? s1 : s2 >> 4) & mA) | ((s1 >> 2) & mB);
                 if constexpr (RT == 1) {  // lane group q: sub-blocks 2q, 2q + 1
-                    *reinterpret_cast<u32x2 *>(stab + buf * L::ST + l16 * gemm::SROW + 8 * q) = pairs(d, nm, sc >> qsh, mn >> qsh, 0);
+                    *reinterpret_cast<u32x2 *>(stab + buf * L::ST + l16 * gemm::SROW + 8 * q) = pairs(d, nm, sc >> qsh, mn >> qsh, B0{});
                 } else {  // half-wavefront h: sub-blocks 4h .. 4h + 3
                     u32x2 *dst = reinterpret_cast<u32x2 *>(stab + buf * L::ST + (lane & 31) * gemm::SROW + 16 * (lane >> 5));
-                    dst[0] = pairs(d, nm, sc, mn, 0);
-                    dst[1] = pairs(d, nm, sc, mn, 16);
+                    dst[0] = pairs(d, nm, sc, mn, B0{});
+                    dst[1] = pairs(d, nm, sc, mn, B2{});
                 }
             } else {
                 const int row = min(64 * k + lane, 16 * RT - 1);
                 u32x2 *dst = reinterpret_cast<u32x2 *>(stab + buf * L::ST + row * gemm::SROW);
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    dst[j] = pairs(d, nm, scales4(j >> 1, s0, s2), mins4(j >> 1, s1, s2), 16 * (j & 1));
+                for (int j = 0; j < 2; ++j) {
+                    const uint32_t sc = scales4(j, s0, s2), mn = mins4(j, s1, s2);
+                    dst[2 * j] = pairs(d, nm, sc, mn, B0{});
+                    dst[2 * j + 1] = pairs(d, nm, sc, mn, B2{});
+                }
             }
         }
-        return __any(any != 0);
+        return __any(any);
     };
     // 2^x of row 16 i + 4 q + v, x from the lane that decodes the row
     auto row_pow2 = [&](const int(&x)[HD], int i, int add, int sign) __attribute__((always_inline)) {
