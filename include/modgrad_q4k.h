@@ -198,6 +198,13 @@ hipError_t launch_matvec_q4k_batched_noalloc(const unsigned char *w_q4, const fl
 hipError_t launch_gemm_q4k_f16(const unsigned char *w_q4, const uint16_t *a_f16, float *c,
                                int out_dim, int blocks_per_row, int m_tokens,
                                hipStream_t stream);
+/* The tile shape that launch_gemm_q4k_f16 picks for such a call on a device of
+ * n_cus compute units: its W rows, tokens and shares of K (host only, launches
+ * nothing). Returns the shape's index, counted from 0 in the order of size, the
+ * last one being that of rows longer than 2^27 values; -1 for invalid
+ * arguments. */
+int mgq_gemm_tile(int out_dim, int blocks_per_row, int m_tokens, int n_cus, int *rows, int *tokens,
+                  int *k_shares);
 
 /* ---------------------------------------------------------------------------
  * Decode glue (kernels/rms_norm.hip, kernels/transformer_ops.hip) and its

@@ -42,6 +42,7 @@ SIGNATURES = {
     "launch_matvec_q4k_batched": (I, [P, P, P, I, I, I, P, S, P]),
     "launch_matvec_q4k_batched_noalloc": (I, [P, P, P, I, I, I, P]),
     "launch_gemm_q4k_f16": (I, [P, P, P, I, I, I, P]),
+    "mgq_gemm_tile": (I, [I, I, I, I, P, P, P]),
     "launch_quantize_matvec_q4k_dp4a_ex": (I, [P, P, P, I, I, P]),
     "launch_rms_norm": (I, [P, P, P, I, I, F]),
     "launch_rms_norm_ex": (I, [P, P, P, I, I, F, P]),

@@ -191,6 +191,13 @@ hipError_t launch_gemm_q4k_f16(const unsigned char *w_q4, const uint16_t *a_f16,
     return mgq::gemm_f16_launch(w_q4, a_f16, c, out_dim, blocks_per_row, m_tokens, stream);
 }
 
+int mgq_gemm_tile(int out_dim, int blocks_per_row, int m_tokens, int n_cus, int *rows, int *tokens,
+                  int *k_shares) {
+    if (out_dim <= 0 || blocks_per_row <= 0 || m_tokens <= 0 || n_cus <= 0 || !rows || !tokens || !k_shares)
+        return -1;
+    return mgq::gemm_tile_shape(out_dim, blocks_per_row, m_tokens, n_cus, rows, tokens, k_shares);
+}
+
 // ------------------------------------------------------ decode-step chain --
 
 struct mgq_chain {

@@ -7,7 +7,7 @@
 // powers of two) rounded to f16 and the weight computed and rounded once in
 // f16; C is scaled back exactly.
 //
-// One kernel, gemm_q4k_f16_kernel, in tile shapes from 32 rows x 32 tokens to
+// One kernel, gemm_q4k_f16_kernel, in tile shapes from 32 rows x 16 tokens to
 // 336 x 128 (kTiles), picked per call by a model of the time of each
 // (gemm_f16_launch).
 //
@@ -22,10 +22,11 @@
 //     every weight is dequantized once per tile, and W never goes through
 //     LDS.
 //   * The loader copies the tokens' 128-value half blocks from memory
-//     straight into LDS (global_load_lds, no registers), NBUF - 1 half blocks
-//     ahead. It issues no other vector memory operation, so its vmcnt waits
-//     are exact (a register spilled around them would make them stricter);
-//     the compute wavefronts' loads are waited for by the compiler.
+//     straight into LDS (global_load_lds, no registers): NBUF half blocks
+//     before the first product, then NBUF - 1 ahead. It issues no other
+//     vector memory operation, so its vmcnt waits are exact (a register
+//     spilled around them would make them stricter); the compute wavefronts'
+//     loads are waited for by the compiler.
 //   * The two wavefronts of a SIMD run a half block's dequantization and
 //     products in opposite orders (run), so that one's vector work falls under
 //     the other's matrix work: 3584 x 18944 at 512 tokens 105 -> 95 us, at 4096
@@ -69,8 +70,6 @@
 // at most. C is multiplied by 2^(20-e) at the end.
 #include "q4k_device.hpp"
 #include "q4k_launch.hpp"
-
-#include <cstdlib>
 
 namespace mgq {
 
@@ -635,7 +634,8 @@ static const GemmTile kTiles[] = {
     MGQ_TILE(3, 8, 7, 1, 2, 1, 7.7f, 3.69f),   // 336 x 128
 };
 #undef MGQ_TILE
-// Rows so long that a tile's offsets pass 32 bits (K above ~16 million).
+constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
+// Rows so long that the offsets inside any tile pass 32 bits (K above 2^27).
 static constexpr auto launch_wide = launch_tile<1, 2, 2, 4, 4, 1, uint64_t>;
 
 hipError_t gemm_prepare() {
@@ -645,24 +645,38 @@ hipError_t gemm_prepare() {
     return e;
 }
 
-hipError_t gemm_f16_launch(const uint8_t *w, const uint16_t *a, float *c, int n, int bpr,
-                           int m_tokens, hipStream_t stream) {
-    if ((uintptr_t)a & 1u) return hipErrorInvalidValue;
-    const long cus = device_cus();
-    const GemmTile *best = nullptr;
+// The shape of a call: an index of kTiles, or kNumTiles for launch_wide.
+static int gemm_pick(int n, int bpr, int m_tokens, long cus) {
+    int best = kNumTiles;
     float best_us = 0.0f;
-    for (const GemmTile &t : kTiles) {
+    for (int i = 0; i < kNumTiles; ++i) {
+        const GemmTile &t = kTiles[i];
         // offsets of a tile's rows and tokens are 32-bit
         if ((int64_t)t.bn * bpr * kBlockBytes > 0xFFFFFFFFll || (int64_t)t.bm * bpr * kBlockElems * 2 > 0xFFFFFFFFll)
             continue;
         const long tiles = (long)((n + t.bn - 1) / t.bn) * ((m_tokens + t.bm - 1) / t.bm);
         const float us = (float)((tiles + cus - 1) / cus) * (t.fixed_us + t.block_us * (float)((bpr + t.nwk - 1) / t.nwk));
-        if (!best || us < best_us) {
-            best = &t;
+        if (best == kNumTiles || us < best_us) {
+            best = i;
             best_us = us;
         }
     }
-    return (best ? best->launch : launch_wide)(w, a, c, n, bpr, m_tokens, stream);
+    return best;
+}
+
+int gemm_tile_shape(int n, int bpr, int m_tokens, int cus, int *rows, int *tokens, int *k_shares) {
+    const int i = gemm_pick(n, bpr, m_tokens, cus);
+    *rows = i < kNumTiles ? kTiles[i].bn : 32;
+    *tokens = i < kNumTiles ? kTiles[i].bm : 32;
+    *k_shares = i < kNumTiles ? kTiles[i].nwk : 4;
+    return i;
+}
+
+hipError_t gemm_f16_launch(const uint8_t *w, const uint16_t *a, float *c, int n, int bpr,
+                           int m_tokens, hipStream_t stream) {
+    if ((uintptr_t)a & 1u) return hipErrorInvalidValue;
+    const int i = gemm_pick(n, bpr, m_tokens, device_cus());
+    return (i < kNumTiles ? kTiles[i].launch : launch_wide)(w, a, c, n, bpr, m_tokens, stream);
 }
 
 }  // namespace mgq

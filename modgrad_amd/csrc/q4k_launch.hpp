@@ -158,9 +158,9 @@ hipError_t dequant_launch(const uint8_t *q, int n_blocks, float *out, hipStream_
 // layout (k % 256 == 0) when the fast kernel does not apply.
 hipError_t gemv_generic_launch(const uint8_t *w, const float *x, float *y, int n, int k,
                                hipStream_t stream);
-// Flat-stream layout with k % 32 == 0 (whole sub-blocks per row), w and x
-// 16-byte aligned; hipErrorNotSupported otherwise (then: generic). A bias (n
-// floats, or null) is added to the row sums.
+// Flat-stream layout with k % 32 == 0 (whole sub-blocks per row), w at any
+// byte and x at any float; hipErrorNotSupported otherwise (then: generic). A
+// bias (n floats, or null) is added to the row sums.
 hipError_t gemv_flat_launch(const uint8_t *w, const float *x, float *y, int n, int k,
                             hipStream_t stream, const float *bias = nullptr);
 
@@ -270,5 +270,7 @@ hipError_t gemm_f16_launch(const uint8_t *w, const uint16_t *a, float *c, int n,
                            int m_tokens, hipStream_t stream);
 // LDS attribute of the GEMM kernel in every tile shape (safe to call often).
 hipError_t gemm_prepare();
+// The tile shape such a call takes on a device of `cus` CUs (host only).
+int gemm_tile_shape(int n, int bpr, int m_tokens, int cus, int *rows, int *tokens, int *k_shares);
 
 }  // namespace mgq

@@ -217,8 +217,8 @@ def test_gemm_operands_at_offsets(L, orc, woff, aoff):
                                                 (20000, 14, 512, 1, 2), (20000, 14, 512, 12, 6),
                                                 (20000, 14, 512, 0, 8)])
 def test_gemm_prefill_shapes_at_offsets(L, orc, n, bpr, m, woff, aoff):
-    # Shapes that take the LDS-dequant kernel when W and A are 16-byte
-    # aligned; misaligned operands must still give the oracle's result.
+    # Large shapes, whose aligned activations are copied straight into LDS;
+    # misaligned operands must still give the oracle's result.
     note(f"gemm prefill-sized n={n} bpr={bpr} m={m}, w offset {woff}, A offset {aoff}")
     rng = np.random.default_rng(n + 7 * m + woff + 131 * aoff)
     w = random_q4k_bytes(rng, n * bpr)

@@ -1,6 +1,7 @@
-"""The prefill GEMM's tile shapes: one case or more for each, at their edges
-(one row, one token, a tile's rows and tokens +- 1, K shares with and without
-a block), pointers of the smallest alignment, and recording into a graph.
+"""The prefill GEMM's tile shapes: cases for each, at their edges (one row, one
+token, a tile's rows and tokens +- 1, K shares with and without a block) and
+over several rounds of their buffers, rows past 32-bit offsets, pointers of
+the smallest alignment, and recording into a graph.
 
 Bounds as for the other GEMM tests: f16 weights (three roundings of 2^-11
 each) keep the Frobenius error below 1e-3 and each element within
@@ -50,24 +51,59 @@ def check(L, orc, n, bpr, m, woff=0, aoff=0, coff=0):
     assert np.linalg.norm(C - C_ref) <= 1e-3 * np.linalg.norm(C_ref)
 
 
-@pytest.mark.parametrize("n,bpr,m", [
-    (1, 1, 1), (17, 3, 16), (33, 5, 15), (1000, 6, 17),           # 32 x 16, four K shares
-    (1000, 1, 129), (4001, 9, 33),                                # 32 x 32
-    (2001, 1, 129), (8003, 5, 33),                                # 32 x 48
-    (16001, 1, 1), (16001, 3, 49), (4001, 3, 129),                # 64 x 48, two K shares
-    (8003, 2, 97), (16001, 3, 81),                                # 64 x 80
-    (20479, 2, 1), (30001, 2, 47),                                # 128 x 48
-    (30001, 1, 49), (16001, 3, 97),                               # 128 x 64
-    (16001, 2, 129), (30001, 1, 79),                              # 128 x 80
-    (20479, 1, 17), (30001, 3, 47),                               # 160 x 48
-    (37888, 26, 33),                                              # 160 x 48, two K shares
-    (20479, 2, 127), (20479, 3, 97),                              # 160 x 80
-    (56001, 4, 100), (7001, 4, 1021),                             # 224 x 128
-    (60001, 2, 1), (85007, 3, 79), (42001, 1, 5), (42001, 3, 127),  # 336 x 80
-    (30001, 1, 161), (85007, 2, 81), (60001, 3, 127)])            # 336 x 128
+# rows, tokens and K shares of a tile -> the cases that take it on 256 CUs
+# (asserted by tests/test_gemm_tile_pick.py): at its edges, and last one of
+# 4 to 17 blocks whose token buffers, register sets and scale tables all come
+# round again in every K share, the shares unequal
+CASES = {
+    (32, 16, 4): [(1, 1, 1), (17, 3, 16), (33, 5, 15), (1000, 6, 17), (33, 29, 15)],
+    (32, 32, 4): [(1000, 1, 129), (4001, 9, 33), (806, 13, 149)],
+    (32, 48, 4): [(8003, 5, 33), (1032, 13, 225)],
+    (64, 48, 2): [(2001, 1, 129), (16001, 1, 1), (4001, 3, 129), (1168, 11, 291)],
+    (64, 80, 2): [(8003, 2, 97), (16001, 3, 49), (1852, 11, 388)],
+    (128, 48, 2): [(20479, 2, 1), (16001, 3, 81), (30001, 2, 47), (30001, 3, 47), (60001, 2, 1),
+                   (3344, 7, 325)],
+    (128, 64, 2): [(30001, 1, 49), (16001, 3, 97), (3238, 7, 436)],
+    (128, 80, 2): [(16001, 2, 129), (30001, 1, 79), (4695, 7, 389)],
+    (160, 48, 1): [(20479, 1, 17), (6660, 7, 269)],
+    (160, 48, 2): [(37888, 26, 33), (5458, 17, 321)],
+    (160, 80, 2): [(20479, 2, 127), (20479, 3, 97), (5387, 7, 416)],
+    (224, 128, 1): [(56001, 4, 100), (7001, 4, 1021), (13156, 4, 489)],
+    (336, 80, 1): [(85007, 3, 79), (42001, 1, 5), (42001, 3, 127), (6301, 4, 489)],
+    (336, 128, 1): [(30001, 1, 161), (85007, 2, 81), (60001, 3, 127), (14360, 5, 416)],
+}
+
+
+@pytest.mark.parametrize("n,bpr,m", [c for cases in CASES.values() for c in cases])
 def test_gemm_tile_shapes(L, orc, n, bpr, m):
     note(f"gemm tiles n={n} bpr={bpr} m={m}")
     check(L, orc, n, bpr, m)
+
+
+def test_gemm_rows_past_32_bit_offsets(L):
+    # 2^27 values a row: offsets inside a tile pass 32 bits (64-bit ones then).
+    # The weights of the last 64 blocks of every row are the only nonzero ones,
+    # so the reference is that of a 64-block product.
+    import torch
+    n, bpr, m, tail = 3, 524288, 2, 64
+    note(f"gemm n={n} bpr={bpr} m={m}")
+    rng = np.random.default_rng(27)
+    w = torch.zeros((n, bpr, 144), dtype=torch.uint8, device="cuda")
+    wt = random_q4k_bytes(rng, n * tail)
+    w[:, -tail:] = dev(wt).view(n, tail, 144)
+    a = torch.ones((m, bpr * 256), dtype=torch.float16, device="cuda")
+    at = rng.standard_normal((m, tail * 256)).astype(np.float16)
+    a[:, -tail * 256:] = torch.from_numpy(at).cuda()
+    ct = empty_f32(m * n)
+    _lib.check("gemm", L.launch_gemm_q4k_f16(ptr(w), ptr(a), ptr(ct), n, bpr, m, None))
+    got = host(ct).reshape(m, n)
+    ws, as_, small = dev(wt), dev(at.view(np.uint16)), empty_f32(m * n)
+    _lib.check("gemm", L.launch_gemm_q4k_f16(ptr(ws), ptr(as_), ptr(small), n, tail, m, None))
+    # the same weights, rounded the same (a row's exponent starts at its first
+    # nonzero block): only the order of the f32 sums differs, by K shares
+    want = host(small).reshape(m, n)
+    assert np.all(np.isfinite(got)) and np.linalg.norm(want) > 0
+    assert np.linalg.norm(got - want) <= 2e-6 * np.linalg.norm(want)
 
 
 # weights at an odd byte, activations at an odd f16, C at a 4-byte address:
@@ -77,6 +113,14 @@ def test_gemm_tile_shapes(L, orc, n, bpr, m):
 def test_gemm_unaligned_pointers(L, orc, n, bpr, m, woff, aoff, coff):
     note(f"gemm n={n} bpr={bpr} m={m} offsets {woff} {aoff} {coff}")
     check(L, orc, n, bpr, m, woff, aoff, coff)
+
+
+# ... over several rounds of the buffers that those registers go to
+@pytest.mark.parametrize("tile", CASES)
+def test_gemm_unaligned_activations(L, orc, tile):
+    n, bpr, m = CASES[tile][-1]
+    note(f"gemm tile {tile} n={n} bpr={bpr} m={m}, A at +2")
+    check(L, orc, n, bpr, m, 0, 2, 0)
 
 
 CAPTURE = """

@@ -458,10 +458,10 @@ def _gemm_check(L, orc, w, a, n, bpr, m, rows=None):
     assert np.linalg.norm(C - C_ref) <= 1e-3 * np.linalg.norm(C_ref)
 
 
-# (200, 40): the 128-token kernel; (32000, 256): 200 tiles of 160 x 256, the
-# LDS-dequant kernel, one block per row; (20000, 512): the LDS-dequant kernel
-# with 14 blocks per row, where a row's scale follows its blocks (rows
-# sampled on the large shapes)
+# (200, 40): 32 x 16 tiles, one block per K share; (32000, 256): one block per
+# row; (20000, 512): 336 x 128 tiles with 14 blocks per row, where a row's
+# exponent follows its blocks (the other tiles' rescales: test_gpu_gemm_range;
+# rows sampled on the large shapes)
 @pytest.mark.parametrize("n,m", [(200, 40), (32000, 256), (20000, 512)])
 @pytest.mark.parametrize("kind", ["tiny", "huge", "mixed", "rising", "random"])
 def test_gemm_f16_dynamic_range(L, orc, kind, n, m):
@@ -474,9 +474,7 @@ def test_gemm_f16_dynamic_range(L, orc, kind, n, m):
     _gemm_check(L, orc, w, a, n, bpr, m, rows)
 
 
-# The 128-token kernel at its 160-row tile height with several super-blocks
-# (the raw-W LDS refill across super-blocks) and several token tiles:
-# (70000, 3, 16) and the config-5 weight at M = 256 (rows sampled)
+# Many rows at few tokens, and the 18944 x 3584 weight at M = 256 (rows sampled)
 @pytest.mark.parametrize("n,bpr,m", [(70000, 3, 16), (18944, 14, 256)])
 def test_gemm_160_row_tiles_multi_block(L, orc, n, bpr, m):
     note(f"gemm 160-row tiles n={n} bpr={bpr} m={m}")
@@ -488,10 +486,8 @@ def test_gemm_160_row_tiles_multi_block(L, orc, n, bpr, m):
     _gemm_check(L, orc, w, a, n, bpr, m, rows)
 
 
-# Shapes the LDS-dequant kernel takes (one round of 160 x 256 tiles more than
-# half full, or several rounds at least 85 % full): full token tiles, ragged
-# tokens, ragged rows, several super-blocks; two rounds (476 tiles) with full
-# and with ragged token tiles
+# Large calls: full token tiles, ragged tokens, ragged rows, several
+# super-blocks, several rounds of tiles
 @pytest.mark.parametrize("n,bpr,m", [(32000, 1, 256), (30000, 3, 250), (20000, 14, 512),
                                      (18944, 2, 1024), (18944, 2, 1000)])
 def test_gemm_lds_kernel_shapes(L, orc, n, bpr, m):
