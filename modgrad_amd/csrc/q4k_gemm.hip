@@ -606,10 +606,13 @@ static hipError_t launch_tile(const uint8_t *w, const uint16_t *a, float *c, int
 
 // The tile shapes. A work-group of one takes fixed_us + block_us per block of
 // its K share, with every CU holding one; a call takes as many rounds of that
-// as its tiles fill (rounds of all CUs, the last one counted whole). Fitted to
-// 438 shapes (N 576-37888, K 1536-18944, M 17-2048): the predicted best shape
-// is within 0.4 % of the measured best on average, 17 % at worst. W's prefetch
-// is two blocks where the registers allow it without losing a wavefront.
+// as its tiles fill (rounds of all CUs, the last one counted whole). The times
+// rank the shapes, they do not predict a call: large calls take 13-17 %
+// longer. Fitted to 438 shapes (N 576-37888, K 1536-18944, M 17-2048), 32 x 16
+// again on 700 others (N 33-47104, K 1536-26624, M 1-4096): over these the
+// picked shape is within 0.1 % of the best one on average, 7 % at worst.
+// W's prefetch is two blocks where that was faster; 32 x 32 and 32 x 48 would
+// hold two without losing a wavefront, and the same to 1 % with them.
 struct GemmTile {
     int bn, bm, nwk;
     float fixed_us, block_us;
@@ -618,7 +621,7 @@ struct GemmTile {
 #define MGQ_TILE(RT, TT, NWN, NWK, NBUF, PD, FIXED, BLOCK) \
     {16 * RT * NWN, 16 * TT, NWK, FIXED, BLOCK, launch_tile<RT, TT, NWN, NWK, NBUF, PD, uint32_t>}
 static const GemmTile kTiles[] = {
-    MGQ_TILE(1, 1, 2, 4, 4, 2, 1.8f, 1.08f),   //  32 x  16
+    MGQ_TILE(1, 1, 2, 4, 4, 2, 2.2f, 1.12f),   //  32 x  16
     MGQ_TILE(1, 2, 2, 4, 4, 1, 2.2f, 1.43f),   //  32 x  32
     MGQ_TILE(1, 3, 2, 4, 3, 1, 2.4f, 1.68f),   //  32 x  48
     MGQ_TILE(1, 3, 4, 2, 3, 2, 2.7f, 1.31f),   //  64 x  48
