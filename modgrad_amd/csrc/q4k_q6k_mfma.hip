@@ -814,8 +814,11 @@ hipError_t gemv_q6k_mfma_launch(const uint8_t *w, const float *x, float *y, int 
 
 // Q6_K on Q8_1 activations (launch_matvec_q6k_dp4a) on the wave-private
 // kernel. 3584 x 18944: 194 -> 15.9 us, against the byte-loading vector-ALU
-// kernel that serves what this one cannot take (bpr > 91, misaligned or
-// unpadded weights).
+// kernel that serves what this one cannot take: misaligned or unpadded weights,
+// and rows whose table does not fit LDS. A row of more than 14 blocks takes
+// 1120 bytes a block, and 1024 per round of its 16-row groups over the CUs:
+// up to 90 blocks fit for n <= 4096 on 256 CUs, 89 to 8192, 88 to 12288, one
+// less for every 4480 rows or so.
 hipError_t gemv_q6k_q8_mfma_launch(const uint8_t *w, const int8_t *xq, const float *xd, float *y,
                                    int n, int bpr, hipStream_t stream) {
     using namespace q6m;

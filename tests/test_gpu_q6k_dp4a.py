@@ -1,8 +1,8 @@
 """Q6_K matvec on Q8_1 activations (launch_matvec_q6k_dp4a): the matrix-core
 kernel at the edges of its shapes (one block, blocks per wavefront + 1, table
-items per thread, the longest row its LDS takes and the one past it, ragged
-row groups), int8 activations at any byte, the extreme int8 values, and a
-non-finite scale.
+items per thread, the longest row that its LDS takes and the one past it: 90
+blocks up to 4096 rows on 256 CUs, 89 above; ragged row groups), int8
+activations at any byte, the extreme int8 values, and a non-finite scale.
 
 Bound: the integer dots are exact, so y differs from the oracle's float
 evaluation only by the f32 rounding of its terms and their sum: 2^-20 of the
@@ -33,7 +33,8 @@ def run(orc, n, bpr, xq, xd, xoff=0, woff=0):
 
 
 @pytest.mark.parametrize("n,bpr", [(8, 1), (24, 3), (136, 13), (40, 14), (48, 15), (16, 16), (520, 17),
-                                   (24, 32), (24, 33), (3584, 74), (16, 64), (16, 65), (16, 91), (16, 92),
+                                   (24, 32), (24, 33), (3584, 74), (16, 64), (16, 65), (16, 90),
+                                   (4096, 90), (4112, 90), (16, 91), (16, 92),
                                    (9600, 16), (70000, 2), (17, 8), (33, 5)])
 def test_q6k_dp4a_shapes(orc, n, bpr):
     note(f"q6k dp4a n={n} bpr={bpr}")
