@@ -460,12 +460,14 @@ def _gemm_check(L, orc, w, a, n, bpr, m, rows=None):
 
 # (200, 40): 32 x 16 tiles, one block per K share; (32000, 256): one block per
 # row; (20000, 512): 336 x 128 tiles with 14 blocks per row, where a row's
-# exponent follows its blocks (the other tiles' rescales: test_gpu_gemm_range;
-# rows sampled on the large shapes)
-@pytest.mark.parametrize("n,m", [(200, 40), (32000, 256), (20000, 512)])
+# exponent follows its blocks (rows sampled on the large shapes);
+# and rescales in the other tiles: (201, 40) 32 x 16 with five blocks per K
+# share, (4608, 512) 128 x 80 and (18944, 256) 336 x 80 in both orders of the
+# paired wavefronts
+@pytest.mark.parametrize("n,m", [(200, 40), (32000, 256), (20000, 512), (201, 40), (4608, 512), (18944, 256)])
 @pytest.mark.parametrize("kind", ["tiny", "huge", "mixed", "rising", "random"])
 def test_gemm_f16_dynamic_range(L, orc, kind, n, m):
-    bpr = {200: 4, 32000: 1, 20000: 14}[n]
+    bpr = {200: 4, 201: 20, 32000: 1}.get(n, 14)
     note(f"gemm range {kind} n={n} bpr={bpr} m={m}")
     rng = np.random.default_rng(0x6E11 + m)
     w = _range_weight(rng, n, bpr, kind)
